@@ -9,14 +9,17 @@
 //
 // Here, too, one lane owns one column and both sweeps run in one launch, with the k-caches (u_stage ring,
 // wcon at k and k+1, ccol/dcol at k-1, data_col at k+1) in VGPRs.  The forward sweep's ccol/dcol for the
-// backward sweep are kept on chip when nk allows it (see the ONCHIP variant), otherwise they go to a
-// per-launch scratch buffer in the k-major layout the lanes read coalesced.
+// backward sweep are kept on chip as far as it holds them (up to 80 levels vadv_onchip_kernel and its persistent and
+// 16-byte-request forms, deeper columns vadv_deep_kernel: registers, then LDS, then scratch).  Fields that span 4 GiB
+// or more, past the 32-bit buffer offsets, take vadv_scratch_kernel: ccol/dcol in a per-launch scratch buffer in the
+// k-major layout the lanes read coalesced.
 // Arithmetic follows the functors operation by operation (built with -ffp-contract=off).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <mutex>
 
+#include "column.hpp"
 #include "common.hpp"
 #include "functors.hpp"
 #include "tuning.hpp"
@@ -867,6 +870,47 @@ namespace gt355 {
             }
         }
 
+        // Columns deeper than the register buckets: the persistent grid of vadv_persist_kernel over column.hpp's sweep,
+        // ccol/dcol of R + TL levels on chip.  Each wavefront takes strips with a static stride and starts the next
+        // strip's first D levels of loads NB levels before the end of a strip's backward sweep.
+        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK>
+        __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+        vadv_deep_kernel(ST *__restrict__ uts_f, const ST *__restrict__ us_f, const ST *__restrict__ wc_f,
+            const ST *__restrict__ up_f, const ST *__restrict__ ut_f, CT dtr, int ni, int nk, int64_t sj, int64_t sk,
+            int64_t wsj, int64_t wsk, int strips_i, int nitems, int nxcd, CT *scratch, int tail_rows) {
+            __shared__ ST s_up[PARK ? R : 1][64];
+            __shared__ CT s_tail[TL > 0 ? TL * 128 : 1];
+            column_src f{make_rsrc(uts_f), make_rsrc(us_f), make_rsrc(wc_f), make_rsrc(up_f), make_rsrc(ut_f),
+                (uint32_t)(sk * (int64_t)sizeof(ST)), (uint32_t)(wsk * (int64_t)sizeof(ST)), nk};
+            const rsrc_t sc = make_rsrc(scratch + (int64_t)blockIdx.x * tail_rows * 128);
+            // the lane's byte offsets in strip `it` (lanes past ni take column ni-1)
+            auto offsets = [&](int it, uint32_t &cb, uint32_t &wb) {
+                const int si = it % strips_i, j = it / strips_i;
+                const int i = min(si * 64 + (int)threadIdx.x, ni - 1);
+                cb = (uint32_t)(((int64_t)j * sj + i) * (int64_t)sizeof(ST));
+                wb = (uint32_t)(((int64_t)j * wsj + i) * (int64_t)sizeof(ST));
+            };
+            int it = xcd_remap(blockIdx.x, gridDim.x, nxcd);
+            if (it >= nitems)
+                return; // a whole wavefront leaves; there is no barrier in this kernel
+            column_sweep<ST, CT, R, D, TL, NB, PARK> sw;
+            uint32_t cb, wb;
+            offsets(it, cb, wb);
+            sw.prologue(f, cb, wb);
+            for (; it < nitems; it += gridDim.x) {
+                const int nx = it + (int)gridDim.x;
+                uint32_t ncb = cb, nwb = wb;
+                sw.sweep(f, dtr, cb, wb, s_up, s_tail, sc, [&]() {
+                    if (nx < nitems) {
+                        offsets(nx, ncb, nwb);
+                        sw.prologue(f, ncb, nwb);
+                    }
+                });
+                cb = ncb;
+                wb = nwb;
+            }
+        }
+
         // Largest linear element offset of a field's allocation box (lower/upper are the box around the origin).
         inline int64_t alloc_last(const gt355_field *f) {
             return (int64_t)(f->upper[0] - 1) + (int64_t)(f->upper[1] - 1) * f->stride[1] +
@@ -898,9 +942,71 @@ namespace gt355 {
             return 80;
         }
 
-        // ext_buf == nullptr: the deep-column path takes its ccol/dcol buffer from the per-stream scratch pool.
-        // Otherwise ext_buf (ext_bytes long) is used and nothing is allocated: the rows are processed in chunks whose
-        // ccol/dcol fit it (columns are independent, so a chunked launch computes the same bits).
+        // One instantiation of the deep kernel: a wavefront per SIMD at most, fewer if the scratch of the levels past
+        // R + TL would exceed `budget` bytes (what the all-scratch kernel needs, or the caller's buffer).  Returns
+        // false, launching nothing, if not even a quarter of the wavefronts fit.
+        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK>
+        bool launch_deep_as(const gt355_field *uts, const gt355_field *us, const gt355_field *wc,
+            const gt355_field *up, const gt355_field *ut, CT dtr, int ni, int nj, int nk, hipStream_t stream,
+            void *ext_buf, size_t budget, int *rc) {
+            const int strips_i = (ni + 63) / 64;
+            const int64_t items = (int64_t)strips_i * nj;
+            if (items >= (int64_t(1) << 31))
+                return false;
+            const int tail_rows = nk > R + TL ? (nk - R - TL + D - 1) / D * D : 0;
+            const size_t wave_bytes = (size_t)tail_rows * 128 * sizeof(CT);
+            const int64_t want = std::min<int64_t>(items, (int64_t)cu_count() * 4);
+            const int64_t fit = wave_bytes ? (int64_t)(budget / wave_bytes) : want;
+            const int64_t waves = std::min(want, fit);
+            if (waves < 1 || waves * 4 < want)
+                return false;
+            // the pool's buffer is sized for the all-scratch kernel whatever part of it this split uses, so that one
+            // run outside capture readies the stream for captures of every shape that needs no more
+            void *buf = ext_buf;
+            *rc = GT355_OK;
+            if (!ext_buf && (*rc = scratch_for(stream, budget, &buf)))
+                return true;
+            vadv_deep_kernel<ST, CT, R, D, TL, NB, PARK><<<(int)waves, 64, 0, stream>>>((ST *)uts->origin,
+                (const ST *)us->origin, (const ST *)wc->origin, (const ST *)up->origin, (const ST *)ut->origin, dtr, ni,
+                nk, uts->stride[1], uts->stride[2], wc->stride[1], wc->stride[2], strips_i, (int)items, xcd_count(),
+                (CT *)buf, tail_rows);
+            *rc = check_launch("gt355_vadv");
+            return true;
+        }
+        // The split of a column over registers, LDS and scratch, by storage and compute type and depth: as many
+        // register levels as compile without spills at a load-ahead of 4 (FP64) or 8 levels.  Measured against
+        // vadv_scratch_kernel: FP64 192x160x137 123 -> 39.0 us (202 MB: 5.2 TB/s), 256x256x137 mixed 145 -> 42-45 us,
+        // FP32 118 -> 39.8 us.
+        template <class ST, class CT>
+        bool launch_deep(const gt355_field *uts, const gt355_field *us, const gt355_field *wc, const gt355_field *up,
+            const gt355_field *ut, CT dtr, int ni, int nj, int nk, hipStream_t stream, void *ext_buf, size_t budget,
+            int *rc) {
+#define GT355_DEEP(R, D, TL, NB, PARK)                                                                               return launch_deep_as<ST, CT, R, D, TL, NB, PARK>(                                                                   uts, us, wc, up, ut, dtr, ni, nj, nk, stream, ext_buf, budget, rc)
+            if constexpr (sizeof(CT) == 4) {
+                // 256x256 columns: 85 levels 25.3 us (29.9 with 128 register levels), 100 levels 29.2 (31.1); 120
+                // levels 33.6 us with 128 register levels against 35.0 with 96, 137 levels 39.8 against 43.0
+                if (nk <= 112)
+                    GT355_DEEP(96, 8, 32, 32, true);
+                GT355_DEEP(128, 8, 16, 32, true);
+            } else if constexpr (sizeof(ST) == 4) {
+                // u_pos parked while no more than 16 levels are left for the LDS tail beside it: 256x256x100 29.4 us
+                // against 30.5 re-read; 256x256x120 33.3-35.3 re-read against 37.0 parked (8 levels in scratch), 137
+                // levels 42.1-45.0 against 51.4
+                if (nk <= 112)
+                    GT355_DEEP(96, 8, 16, 32, true);
+                GT355_DEEP(96, 8, 40, 16, false);
+            } else {
+                // 256x256x137 75.3 us; 88 register levels (4 ahead) 78.0, 80 (8 ahead) 85.5; at 100 levels 53.6, 53.3
+                // and 55.7 us
+                GT355_DEEP(96, 4, 40, 24, false);
+            }
+#undef GT355_DEEP
+        }
+
+        // ext_buf == nullptr: a path that needs ccol/dcol scratch takes it from the per-stream scratch pool.
+        // Otherwise ext_buf (ext_bytes long) is used and nothing is allocated: vadv_deep_kernel launches no more
+        // wavefronts than it holds tails for, and vadv_scratch_kernel processes the rows in chunks whose ccol/dcol fit
+        // it (columns are independent, so a chunked launch computes the same bits).
         template <class ST, class CT>
         int launch_vadv(const gt355_field *uts, const gt355_field *us, const gt355_field *wc, const gt355_field *up,
             const gt355_field *ut, double dtr_stage, int ni, int nj, int nk, hipStream_t stream,
@@ -1033,20 +1139,24 @@ namespace gt355 {
             }
             // ccol/dcol of levels 0..nk-2 for every column of a row
             const size_t row_bytes = sizeof(CT) * (size_t)ni * (size_t)(2 * nk - 1);
-            int rows = nj;
+            GT355_CHECK(!ext_buf || row_bytes <= ext_bytes,
+                "gt355_vadv_noalloc: ni = %d, nk = %d needs %zu bytes of ccol/dcol for one row of columns, more "
+                "than the %zu-byte static scratch holds",
+                ni, nk, row_bytes, ext_bytes);
+            int rows = ext_buf ? (int)std::min<size_t>((size_t)nj, ext_bytes / row_bytes) : nj;
+            GT355_CHECK((std::min(rows, nj) + 3) / 4 <= 65535, "gt355_vadv: nj too large");
+            if (fits32) {
+                int rc = GT355_OK;
+                if (launch_deep<ST, CT>(uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, ext_buf,
+                        ext_buf ? ext_bytes : row_bytes * (size_t)nj, &rc))
+                    return rc;
+            }
             void *buf = ext_buf;
-            if (ext_buf) {
-                GT355_CHECK(row_bytes <= ext_bytes,
-                    "gt355_vadv_noalloc: ni = %d, nk = %d needs %zu bytes of ccol/dcol for one row of columns, more "
-                    "than the %zu-byte static scratch holds",
-                    ni, nk, row_bytes, ext_bytes);
-                rows = (int)std::min<size_t>((size_t)nj, ext_bytes / row_bytes);
-            } else {
+            if (!ext_buf) {
                 int rc = scratch_for(stream, row_bytes * (size_t)nj, &buf);
                 if (rc)
                     return rc;
             }
-            GT355_CHECK((std::min(rows, nj) + 3) / 4 <= 65535, "gt355_vadv: nj too large");
             for (int j0 = 0; j0 < nj; j0 += rows) {
                 const int nr = std::min(rows, nj - j0);
                 dim3 grid((ni + 63) / 64, (nr + 3) / 4);
