@@ -10,8 +10,10 @@
 //    grid-stride loop;
 //  * with elements of 4 or 8 bytes, unit strides along a (source) and b (destination) and aligned vectors, the
 //    tiles move 16 bytes per access on both sides (lt_tile_vec_kernel);
+//  * where one of the two extents is short (a field's k levels), tiles that hold it whole, each side 16 bytes per
+//    access where its own rows are aligned (lt_run_kernel);
 //  * a == b: a flat copy along a, 256 elements per workgroup row, the outer index decomposed once per row.
-// Elements are moved as raw words of 1, 2, 4, 8 or 16 bytes, with non-temporal loads and stores.
+// Elements are moved as raw words of 1, 2, 4, 8 or 16 bytes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -164,6 +166,96 @@ namespace gt355 {
             }
         }
 
+        // The transpose with a tile of run-time extents, one of which is the whole extent of its dimension: a
+        // dimension of at most LT_RUN elements (the k levels of a field) becomes one run per row, so that the side on
+        // which it is contiguous moves whole runs, and the partial lines at a run's ends belong to neighbouring runs
+        // of neighbouring tiles, which the same XCD's L2 merges (default cache policy there).  Splitting it into 16 or
+        // 64 elements instead makes every piece of an unaligned row two partial lines.  The other dimension is cut into
+        // whole 128-byte lines.  VA / VB: elements per access along a on the source side and along b on the destination
+        // side, 1 or 16 bytes' worth, each by that side's own alignment; the end of a row that is no whole vector moves
+        // element by element.  Loads go UN at a time into registers before they are written to LDS.  ma / mb: the
+        // multipliers (lt_div) of the accesses per tile row (ta / VA) and column (tb / VB).
+        constexpr int LT_RUN = 160;
+        // e / n by the multiplier ceil(2^32 / n) (0 stands for n = 1, whose multiplier does not fit)
+        __device__ __forceinline__ int lt_div(int e, uint32_t m) { return m ? (int)__umulhi((uint32_t)e, m) : e; }
+        template <class W, int VA, int VB, bool NT>
+        __global__ void __launch_bounds__(256) lt_run_kernel(W *__restrict__ dst, const W *__restrict__ src, lt_desc d,
+            int ta, int tb, uint32_t ma, uint32_t mb, uint32_t tiles_a, uint32_t tiles_b, int ntiles, int nxcd) {
+            extern __shared__ __align__(16) char lt_smem[];
+            W *tile = (W *)lt_smem; // [tb][ta + 1 - ta % 2]: an odd row length keeps column reads off one bank
+            typedef W veca __attribute__((ext_vector_type(VA)));
+            typedef W vecb __attribute__((ext_vector_type(VB)));
+            const int ld = ta | 1;
+            constexpr int UN = VA == 1 ? 8 : 4;
+            const int t = xcd_remap(blockIdx.x, ntiles, nxcd);
+            const uint32_t it_a = (uint32_t)t % tiles_a, r = (uint32_t)t / tiles_a, it_b = r % tiles_b;
+            int64_t so, dof;
+            outer_offsets<uint32_t>(d, r / tiles_b, so, dof);
+            const int64_t a0 = (int64_t)it_a * ta, b0 = (int64_t)it_b * tb;
+            const int ea = (int)min((int64_t)ta, d.dims[d.a] - a0), eb = (int)min((int64_t)tb, d.dims[d.b] - b0);
+            const int64_t ssa = d.ss[d.a], ssb = d.ss[d.b], dsa = d.ds[d.a], dsb = d.ds[d.b];
+            const W *sp = src + so + a0 * ssa + b0 * ssb;
+            W *dp = dst + dof + a0 * dsa + b0 * dsb;
+            const int na = (ta + VA - 1) / VA, n = na * tb; // vectors per row, accesses
+            for (int e0 = threadIdx.x; e0 < n; e0 += 256 * UN) {
+                W v[UN][VA];
+#pragma unroll
+                for (int q = 0; q < UN; ++q) {
+                    const int e = e0 + 256 * q;
+                    const int bb = lt_div(e, ma), aa = (e - bb * na) * VA;
+                    if (e < n && bb < eb) {
+                        if (VA > 1 && aa + VA <= ea) {
+                            const veca *q16 = (const veca *)(sp + aa + bb * ssb);
+                            const veca w = NT ? __builtin_nontemporal_load(q16) : *q16;
+#pragma unroll
+                            for (int x = 0; x < VA; ++x)
+                                v[q][x] = w[x];
+                        } else {
+#pragma unroll
+                            for (int x = 0; x < VA; ++x)
+                                if (aa + x < ea)
+                                    v[q][x] = sp[(aa + x) * ssa + bb * ssb];
+                        }
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < UN; ++q) {
+                    const int e = e0 + 256 * q;
+                    const int bb = lt_div(e, ma), aa = (e - bb * na) * VA;
+                    if (e < n) {
+#pragma unroll
+                        for (int x = 0; x < VA; ++x)
+                            if (VA == 1 || aa + x < ta)
+                                tile[bb * ld + aa + x] = v[q][x];
+                    }
+                }
+            }
+            __syncthreads();
+            const int nb = (tb + VB - 1) / VB, m = nb * ta;
+#pragma unroll 4
+            for (int e = threadIdx.x; e < m; e += 256) {
+                const int aa = lt_div(e, mb), bb = (e - aa * nb) * VB;
+                if (aa >= ea)
+                    continue;
+                if (VB > 1 && bb + VB <= eb) {
+                    vecb w;
+#pragma unroll
+                    for (int x = 0; x < VB; ++x)
+                        w[x] = tile[(bb + x) * ld + aa];
+                    vecb *q16 = (vecb *)(dp + aa * dsa + bb);
+                    if constexpr (NT)
+                        __builtin_nontemporal_store(w, q16);
+                    else
+                        *q16 = w;
+                } else {
+#pragma unroll
+                    for (int x = 0; x < VB; ++x)
+                        if (bb + x < eb)
+                            dp[aa * dsa + (bb + x) * dsb] = tile[(bb + x) * ld + aa];
+                }
+            }
+        }
+
         template <class W, class IT>
         __global__ void __launch_bounds__(256) lt_flat_kernel(W *__restrict__ dst, const W *__restrict__ src, lt_desc d,
             int64_t outer) {
@@ -191,13 +283,72 @@ namespace gt355 {
                 const int tbsel = sizeof(W) > 8 ? 32 : waste_ok(64) ? 64 : waste_ok(32) ? 32 : 16;
                 // 16-byte accesses: 4- and 8-byte elements, unit stride along a (source) and b (destination), and
                 // every vector aligned: the bases and all strides but those two in multiples of 16 bytes
+                const bool vec_on = tune_param("layout_vec", 1) != 0;
                 bool vec_ok = (sizeof(W) == 4 || sizeof(W) == 8) && d.ss[d.a] == 1 && d.ds[d.b] == 1 &&
-                              (uintptr_t)src % 16 == 0 && (uintptr_t)dst % 16 == 0 && tune_param("layout_vec", 1) != 0;
+                              (uintptr_t)src % 16 == 0 && (uintptr_t)dst % 16 == 0 && vec_on;
                 for (int q = 0; q < d.nd && vec_ok; ++q) {
                     if (q != d.a)
                         vec_ok = (d.ss[q] * (int64_t)sizeof(W)) % 16 == 0;
                     if (q != d.b && vec_ok)
                         vec_ok = (d.ds[q] * (int64_t)sizeof(W)) % 16 == 0;
+                }
+                // a dimension of at most LT_RUN elements: whole runs along it, unless it fills 64-wide tiles and every
+                // row is aligned (measured both ways, a field to dense k-fastest and back, us run / 64 x TB tiles:
+                // FP64 197x261x73 27.9 / 50.7, 256x256x80 35.9 / 45.7, 500x500x20 35 / 88, 256x256x64 28.1 / 27.4;
+                // FP32 256x256x80 18.7 / 30.1, 512x512x136 122 / 230, 256x256x128 30.5 / 28.1)
+                if constexpr (sizeof(W) <= 8) {
+                    const int64_t na = d.dims[d.a], run = std::min(na, nb);
+                    if (run <= LT_RUN && narrow && !(vec_ok && run % 64 == 0)) {
+                        // the other dimension: lines of 128 bytes, as many as make a tile of about 1024 elements (a
+                        // shorter tile leaves a workgroup of 256 idle: 500x500x20 FP64 80 us with one line, 35 with
+                        // four; longer ones take more LDS: 197x261x73 28.4, 29.9, 35.0 us with 16, 32, 64 elements)
+                        constexpr int A = 128 / (int)sizeof(W), V = sizeof(W) >= 4 ? 16 / (int)sizeof(W) : 1;
+                        const int cut = (int)std::min<int64_t>(
+                            std::max(na, nb), A * ((1024 + A * run - 1) / (A * run)));
+                        const int ta = na <= nb ? (int)run : cut, tb = na <= nb ? cut : (int)run;
+                        const int64_t tiles_a = (na + ta - 1) / ta, tiles_b = (nb + tb - 1) / tb,
+                                      ntiles = tiles_a * tiles_b * outer;
+                        // 16-byte accesses on a side whose tile rows all start 16-byte aligned
+                        auto side = [&](const void *p, const int64_t *st, int unit, int ext, int64_t full) {
+                            if (V == 1 || !vec_on || st[unit] != 1 || (uintptr_t)p % 16 || (ext < full && ext % V))
+                                return false;
+                            for (int q = 0; q < d.nd; ++q)
+                                if (q != unit && d.dims[q] > 1 && (st[q] * (int64_t)sizeof(W)) % 16)
+                                    return false;
+                            return true;
+                        };
+                        const bool va = side(src, d.ss, d.a, ta, na), vb = side(dst, d.ds, d.b, tb, nb);
+                        // whole lines of arrays past what the Infinity Cache would keep for the next call are streams
+                        // (301x303x137 FP64 86 -> 73 us non-temporal, 256x256x80 35.9 -> 37.5)
+                        const bool nt = (int64_t)sizeof(W) * na * nb * outer >= (int64_t(64) << 20);
+                        auto magic = [](int n) { return n == 1 ? 0u : (uint32_t)(((uint64_t(1) << 32) + n - 1) / n); };
+                        if (ntiles <= (int64_t(1) << 23)) { // one workgroup per tile
+                            const uint32_t ma = magic(va ? (ta + V - 1) / V : ta), mb = magic(vb ? (tb + V - 1) / V : tb);
+                            const size_t lds = (size_t)(ta | 1) * tb * sizeof(W);
+                            auto run_as = [&](auto va_c, auto vb_c, auto nt_c) {
+                                lt_run_kernel<W, decltype(va_c)::value, decltype(vb_c)::value, decltype(nt_c)::value>
+                                    <<<(int)ntiles, 256, lds, s>>>((W *)dst, (const W *)src, d, ta, tb, ma, mb,
+                                        (uint32_t)tiles_a, (uint32_t)tiles_b, (int)ntiles, xcd_count());
+                            };
+                            auto run_nt = [&](auto va_c, auto vb_c) {
+                                if (nt)
+                                    run_as(va_c, vb_c, std::true_type());
+                                else
+                                    run_as(va_c, vb_c, std::false_type());
+                            };
+                            using one = std::integral_constant<int, 1>;
+                            using vec = std::integral_constant<int, V>;
+                            if (va && vb)
+                                run_nt(vec(), vec());
+                            else if (va)
+                                run_nt(vec(), one());
+                            else if (vb)
+                                run_nt(one(), vec());
+                            else
+                                run_as(one(), one(), std::false_type());
+                            return check_launch("gt355_transform_layout");
+                        }
+                    }
                 }
                 auto go = [&](auto ta_c, auto tb_c) {
                     constexpr int TA = decltype(ta_c)::value, TB = decltype(tb_c)::value;
