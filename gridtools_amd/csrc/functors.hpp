@@ -23,4 +23,18 @@ namespace gt355 {
         return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
     }
 
+    // The same shifts where the edge lanes' values do not matter (they read as zero): no old value to set up.
+    template <int CTRL>
+    __device__ __forceinline__ float dpp_any(float src) {
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, src), CTRL, 0xF, 0xF, true));
+    }
+    template <int CTRL>
+    __device__ __forceinline__ double dpp_any(double src) {
+        const long long s = __builtin_bit_cast(long long, src);
+        const int lo = __builtin_amdgcn_mov_dpp(int(s), CTRL, 0xF, 0xF, true);
+        const int hi = __builtin_amdgcn_mov_dpp(int(s >> 32), CTRL, 0xF, 0xF, true);
+        return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+    }
+
 } // namespace gt355

@@ -168,6 +168,18 @@ namespace gt355 {
                 si_ * 128, sj_ * JB, k);
         }
 
+        // Flat column-pair sweep: one wavefront per 60 outputs of the list of (level, row block, column pair)
+        // (sweep.hpp: hdiff_flat_wave).
+        template <class ST, class CT, int JB, int P, bool ODD>
+        __global__ void __launch_bounds__(256) hdiff_flat_kernel(ST *__restrict__ out, const ST *__restrict__ in,
+            const ST *__restrict__ coeff, hdiff_flat_args g, int waves, int nblocks, int nxcd) {
+            const int w = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, nblocks, nxcd) * 4 + (threadIdx.x >> 6));
+            if (w >= waves)
+                return; // a whole wavefront leaves; there is no barrier in this kernel
+            const rsrc_t r_out = make_rsrc(out);
+            hdiff_flat_wave<ST, CT, JB, P, false, ODD>(r_out, make_rsrc(in), make_rsrc(coeff), r_out, g, w);
+        }
+
         // laplacian.cpp:20-29, one point per thread, one k-level per grid z
         template <class ST, class CT>
         __global__ void __launch_bounds__(256) lap_kernel(ST *__restrict__ out, const ST *__restrict__ in, int ni,
@@ -219,11 +231,57 @@ namespace gt355 {
             return ni % 2 == 0 && ni >= 2 && al(out) && al(in) && al(coeff);
         }
 
+        // Whether the flat pair sweep takes these fields: at least JB rows and two columns, 32-bit byte offsets and
+        // list entries (a last row block's lanes may start up to FLAT_ALIGN pairs past the list).
+        inline bool flat_ok(const gt355_field *out, const gt355_field *in, const gt355_field *coeff, int ni, int nj,
+            int nk, int jb, int64_t es) {
+            auto span = [&](const gt355_field *f, int r) {
+                return ((nk - 1) * f->stride[2] + (nj - 1 + 2 * r) * f->stride[1] + ni + 2 * r) * es;
+            };
+            const int64_t lim = int64_t(1) << 32;
+            return ni >= 2 && nj >= jb && span(in, 2) < lim && span(out, 0) < lim && span(coeff, 0) < lim &&
+                   (int64_t)flat_entries(ni) * ((nj + jb - 1) / jb) * nk < (int64_t(1) << 31) - 64;
+        }
+
+        template <class ST, class CT, int JB, int P>
+        int launch_hdiff_flat(const gt355_field *out, const gt355_field *in, const gt355_field *coeff, int ni,
+            int nj, int nk, hipStream_t stream) {
+            if (!flat_ok(out, in, coeff, ni, nj, nk, JB, sizeof(ST)))
+                return launch_hdiff_sweep<ST, CT, 8, 4>(out, in, coeff, ni, nj, nk, stream);
+            constexpr int64_t S = sizeof(ST);
+            hdiff_flat_args g;
+            g.ni = ni;
+            g.nj = nj;
+            g.np = flat_entries(ni);
+            g.blocks = (nj + JB - 1) / JB;
+            g.osj = (uint32_t)(out->stride[1] * S);
+            g.osk = (uint32_t)(out->stride[2] * S);
+            g.isj = (uint32_t)(in->stride[1] * S);
+            g.isk = (uint32_t)(in->stride[2] * S);
+            g.csj = (uint32_t)(coeff->stride[1] * S);
+            g.csk = (uint32_t)(coeff->stride[2] * S);
+            g.total = g.np * g.blocks * nk;
+            // the list's first and last entries are rim pairs
+            const int waves = (g.total - 2 + FLAT_OW - 1) / FLAT_OW, blocks = (waves + 3) / 4;
+            // `in` is addressed from its lowest read point (-2, -2, 0), so every byte offset is non-negative
+            const ST *in0 = (const ST *)in->origin - 2 - 2 * in->stride[1];
+            if (ni % 2)
+                hdiff_flat_kernel<ST, CT, JB, P, true><<<blocks, 256, 0, stream>>>(
+                    (ST *)out->origin, in0, (const ST *)coeff->origin, g, waves, blocks, xcd_count());
+            else
+                hdiff_flat_kernel<ST, CT, JB, P, false><<<blocks, 256, 0, stream>>>(
+                    (ST *)out->origin, in0, (const ST *)coeff->origin, g, waves, blocks, xcd_count());
+            return check_launch("gt355_hdiff");
+        }
+
         template <class ST, class CT, int JB, int P>
         int launch_hdiff_sweep2(const gt355_field *out, const gt355_field *in, const gt355_field *coeff, int ni,
             int nj, int nk, hipStream_t stream) {
+            // an odd ni or unaligned rows: FP32 storage takes the flat pair sweep (387x251x61 mixed 16.5 us against 19.6
+            // for the one-column sweep), FP64 the one-column sweep (25.2 against 26.0)
             if (!pairs_ok(out, in, coeff, ni, sizeof(ST)))
-                return launch_hdiff_sweep<ST, CT, JB, P>(out, in, coeff, ni, nj, nk, stream);
+                return sizeof(ST) == 4 ? launch_hdiff_flat<ST, CT, 4, 8>(out, in, coeff, ni, nj, nk, stream)
+                                       : launch_hdiff_sweep<ST, CT, JB, P>(out, in, coeff, ni, nj, nk, stream);
             int strips_i = (ni + 127) / 128, strips_j = (nj + JB - 1) / JB;
             int64_t waves = (int64_t)strips_i * strips_j * nk;
             int64_t blocks = (waves + 3) / 4;
@@ -239,7 +297,13 @@ namespace gt355 {
         template <class ST, class CT>
         int launch_cfg(const hdiff_cfg &c, const gt355_field *out, const gt355_field *in, const gt355_field *coeff,
             int ni, int nj, int nk, hipStream_t stream) {
-            if (c.impl == 2) {
+            if (hdiff_is_flat(c)) {
+#define GT355_HFLAT(JB, P)                                                                      \
+    if (c.a == JB && c.b == P)                                                                  \
+        return launch_hdiff_flat<ST, CT, JB, P>(out, in, coeff, ni, nj, nk, stream);
+                GT355_HDIFF_FLATS(GT355_HFLAT)
+#undef GT355_HFLAT
+            } else if (c.impl == 2) {
 #define GT355_HSWEEP2(JB, P)                                                                    \
     if (c.a == JB && c.b == P)                                                                  \
         return launch_hdiff_sweep2<ST, CT, JB, P>(out, in, coeff, ni, nj, nk, stream);
@@ -281,6 +345,9 @@ namespace gt355 {
 #define GT355_ADD_SWEEP2(JB, P) v.push_back({2, JB, P, 0});
             GT355_HDIFF_SWEEPS2(GT355_ADD_SWEEP2)
 #undef GT355_ADD_SWEEP2
+#define GT355_ADD_FLAT(JB, P) v.push_back({2, JB, P, 1});
+            GT355_HDIFF_FLATS(GT355_ADD_FLAT)
+#undef GT355_ADD_FLAT
             return v;
         }
 
@@ -288,7 +355,8 @@ namespace gt355 {
 
     bool hdiff_cfg_instantiated(hdiff_cfg cfg) {
         for (const hdiff_cfg &c : hdiff_candidates())
-            if (c.impl == cfg.impl && c.a == cfg.a && c.b == cfg.b && (cfg.impl != 0 || c.c == cfg.c))
+            if (c.impl == cfg.impl && c.a == cfg.a && c.b == cfg.b && (cfg.impl != 0 || c.c == cfg.c) &&
+                hdiff_is_flat(c) == hdiff_is_flat(cfg))
                 return true;
         return false;
     }
@@ -434,7 +502,7 @@ extern "C" int gt355_tune_hdiff(int precision, const gt355_field *out, const gt3
         const hdiff_cfg &c = cands[ci];
         if (best_of[ci] < win_us)
             win_us = best_of[ci], win = c;
-        if (c.impl == dflt.impl && c.a == dflt.a && c.b == dflt.b && (c.impl != 0 || c.c == dflt.c))
+        if (c.impl == dflt.impl && c.a == dflt.a && c.b == dflt.b && (c.impl == 1 || c.c == dflt.c))
             dflt_us = best_of[ci];
     }
     if (dflt_us <= win_us * 1.02)

@@ -242,4 +242,139 @@ namespace gt355 {
         }
     }
 
+    // Flat column-pair sweep: two adjacent columns per lane and JB rows of one level, as hdiff_pair_wave, but with the
+    // lanes taken from one list over every (level, row block, column pair) instead of from 128-column strips.
+    //
+    // The list of a row block is its pairs from column -2 to ni+1 (one rim pair on each side), padded to NP entries
+    // (a multiple of 4, so that rows of outputs start on whole 32-byte sectors); row blocks follow each other, then
+    // levels.  A wavefront takes 62 consecutive entries (lanes 62 and 63 repeat the pattern unused) and outputs those of
+    // lanes 1..60, so consecutive wavefronts overlap by two rim entries.  A lane's neighbours i-1 and i+2 are always in
+    // the next lanes (DPP shifts): there are no side columns, no scalar loads, no side laplacian and no selects between
+    // sides, and a lane's flx at its left edge is the left lane's flx (a shift instead of a fourth flux).  Rows of any
+    // width fill their lanes, and an odd ni or unaligned rows need no more than the last pair's handling below (a
+    // request only needs element alignment).
+    // What bounds it: ~28 vector instructions per point against ~78 of the one-column sweep (mixed form), so requests:
+    // a wavefront's rows start anywhere, five lines where an aligned 128-column strip has four.  Full strips therefore
+    // stay with hdiff_pair_wave (512x512x80 FP64 95 us against 93-100 here, 1536x1536x80 mixed 403 against 418-450)
+    // and ragged widths come here (mixed, us, strips / flat: 387x251x61 19.6 / 16.5, 130x400x137 26.2 / 19.7,
+    // 101x203x60 8.3 / 5.9).  All JB + 4 = 8 rows are loaded ahead: one memory latency per wavefront.
+    // Rows: block b covers output rows b*JB.., moved up to end at nj (j0 = min(b*JB, nj - JB), nj >= JB); rows that the
+    // block before owns are computed but not stored, so every row has one writer.  Addresses are buffer descriptors
+    // plus a lane offset and one scalar offset per row (the launcher checks that every field spans less than 4 GiB).
+    // Odd ni (ODD): the rim pair on the right starts at ni+1 and would read ni+2, so it is loaded one column to the
+    // left and its a column taken from the second element; the last pair (ni-1, ni) loads coeff one column to the left
+    // and stores its a column alone.
+    constexpr int FLAT_OW = 60, FLAT_ALIGN = 4;
+    struct hdiff_flat_args {
+        int ni, nj, np, blocks;                // np: list entries per row block; blocks: row blocks per level
+        uint32_t osj, osk, isj, isk, csj, csk; // strides in bytes
+        int total;                             // list entries
+    };
+    // list entries per row block
+    inline int flat_entries(int ni) { return ((ni + 1) / 2 + 2 + FLAT_ALIGN - 1) / FLAT_ALIGN * FLAT_ALIGN; }
+    template <class ST, class CT, int JB, int P, bool LAP, bool ODD>
+    __device__ __forceinline__ void hdiff_flat_wave(
+        rsrc_t r_out, rsrc_t r_in, rsrc_t r_co, rsrc_t r_lap, const hdiff_flat_args &g, int w) {
+        constexpr int NR = JB + 4; // in rows j0-2 .. j0+JB+1
+        static_assert(P <= NR, "rows in flight");
+        constexpr uint32_t S = sizeof(ST);
+        const int lane = threadIdx.x & 63;
+        // entry w*OW + lane as (level k, row block b, pair p): the wavefront's first entry by uniform divisions, a
+        // lane's own by carrying over
+        constexpr int OW = FLAT_OW;
+        const int v0 = w * OW;
+        const int q0 = v0 / g.np;
+        int p = v0 - q0 * g.np + lane, k = q0 / g.blocks, b = q0 - k * g.blocks;
+        while (__any(p >= g.np)) {
+            if (p >= g.np) {
+                p -= g.np;
+                if (++b == g.blocks)
+                    b = 0, ++k;
+            }
+        }
+        // the wavefront's last lanes may lie past the list: they repeat its last entry, a rim pair
+        const bool inside = v0 + lane < g.total;
+        if (!inside) {
+            p = g.np - 1;
+            b = g.blocks - 1;
+            k = (g.total / g.np) / g.blocks - 1;
+        }
+        const int pairs = (g.ni + 1) / 2;      // pairs with an output column
+        const int a = 2 * (min(p, pairs + 1) - 1); // the lane's first column (padding entries repeat the rim pair)
+        const int j0 = min(b * JB, g.nj - JB), skip = b * JB - j0;
+        const bool odd_rim = ODD && a > g.ni;       // starts at ni + 1
+        const bool odd_last = ODD && a == g.ni - 1; // its b column is ni
+        const uint32_t vi = (uint32_t)k * g.isk + (uint32_t)j0 * g.isj + (uint32_t)(a + 2 - (odd_rim ? 1 : 0)) * S;
+        // coeff and the outputs exist on [0, ni) only: rim lanes take the nearest pair and store nothing
+        const int ac = min(max(a, 0), 2 * (pairs - 1));
+        const uint32_t vc =
+            (uint32_t)k * g.csk + (uint32_t)j0 * g.csj + (uint32_t)(ac - (ODD && ac == g.ni - 1 ? 1 : 0)) * S;
+        const uint32_t vo = (uint32_t)k * g.osk + (uint32_t)j0 * g.osj + (uint32_t)ac * S;
+        const bool own = inside && lane >= 1 && lane <= OW && p >= 1 && p <= pairs;
+
+        two<ST> rc[P], rk[P];
+        auto load = [&](int t) {
+            rc[t % P] = bload2<ST>(r_in, vi, (uint32_t)t * g.isj); // rim rows are re-read: default cache policy
+            if (t >= 4)
+                rk[t % P] = bload2<ST, CPOL_NT>(r_co, vc, (uint32_t)(t - 4) * g.csj);
+        };
+#pragma clang loop unroll(full)
+        for (int t = 0; t < P; ++t)
+            load(t);
+
+        // rows R-2, R-1, R: columns a and b, in(a-1) and in(b+1); laplacians and fly of the previous rows
+        CT a0 = 0, a1 = 0, a2 = 0, b0 = 0, b1 = 0, b2 = 0, ma1 = 0, pb1 = 0, pb0 = 0;
+        CT la1 = 0, la0 = 0, lb1 = 0, lb0 = 0, flya_m = 0, flyb_m = 0;
+#pragma clang loop unroll(full)
+        for (int t = 0; t < NR; ++t) {
+            const two<ST> v = rc[t % P], kv = rk[t % P];
+            const ST va = odd_rim ? v.b : v.a;
+            if (t + P < NR)
+                load(t + P);
+            a0 = a1; a1 = a2; a2 = CT(va);
+            b0 = b1; b1 = b2; b2 = CT(v.b);
+            const CT ma2 = CT(dpp_any<DPP_WF_SR1>(v.b)), pb2 = CT(dpp_any<DPP_WF_SL1>(va));
+            la0 = la1;
+            lb0 = lb1;
+            if (t >= 2) {
+                // lap of row R-1 at a and b (lap_function, horizontal_diffusion.cpp:41-46)
+                la1 = lap_f<CT>(a1, b1, a2, ma1, a0);
+                lb1 = lap_f<CT>(b1, pb1, b2, a1, b0);
+            }
+            if (t >= 4) {
+                // output row R-2 (horizontal_diffusion.cpp:56-60, 70-74, 86-90)
+                const CT lbp = dpp_any<DPP_WF_SL1>(la0);
+                const CT flx_a = flux_f<CT>(lb0, la0, b0, a0);
+                const CT flx_b = flux_f<CT>(lbp, lb0, pb0, b0);
+                const CT flx_am = dpp_any<DPP_WF_SR1>(flx_b);
+                const CT fly_a = flux_f<CT>(la1, la0, a1, a0);
+                const CT fly_b = flux_f<CT>(lb1, lb0, b1, b0);
+                const CT ka = CT(ODD && odd_last ? kv.b : kv.a), kb = CT(kv.b);
+                const CT ra = a0 - ka * (((flx_a - flx_am) + fly_a) - flya_m);
+                const CT rb = b0 - kb * (((flx_b - flx_a) + fly_b) - flyb_m);
+                flya_m = fly_a;
+                flyb_m = fly_b;
+                if (own && t - 4 >= skip) {
+                    const uint32_t so = (uint32_t)(t - 4) * g.osj;
+                    if (!ODD || !odd_last) {
+                        bstore_pair<ST, CPOL_OUT>(r_out, ST(ra), ST(rb), vo, so);
+                        if constexpr (LAP)
+                            bstore_pair<ST, CPOL_OUT>(r_lap, ST(la0), ST(lb0), vo, so);
+                    } else {
+                        bstore<ST, CPOL_OUT>(r_out, ST(ra), vo, so);
+                        if constexpr (LAP)
+                            bstore<ST, CPOL_OUT>(r_lap, ST(la0), vo, so);
+                    }
+                }
+            } else if (t == 3) {
+                // fly of row j0-1, the fly[j-1] of the first output row
+                flya_m = flux_f<CT>(la1, la0, a1, a0);
+                flyb_m = flux_f<CT>(lb1, lb0, b1, b0);
+            }
+            ma1 = ma2;
+            pb0 = pb1;
+            pb1 = pb2;
+        }
+    }
+
 } // namespace gt355

@@ -101,10 +101,18 @@ namespace gt355 {
     }
 
     hdiff_cfg hdiff_default_cfg(int st_size, int ni) {
-        // measured defaults (MI355X, x80 levels, autotuner winners): FP32 storage takes the column-pair sweep with
+        // measured defaults (MI355X, autotuner winners at x80 levels): FP32 storage takes the column-pair sweep with
         // 8-row strips (256x256: 13.5 us, 512x512: 41 us); FP64 storage the one-column sweep with 8-row strips at
-        // 256x256 (22.2 us) and the column-pair sweep from 512 columns on (88 us against 97 us)
-        return st_size == 4 ? hdiff_cfg{2, 8, 4, 0} : ni >= 512 ? hdiff_cfg{2, 8, 4, 0} : hdiff_cfg{1, 8, 4, 0};
+        // 256x256 (22.2 us) and the column-pair sweep from 512 columns on (88 us against 97 us).  Where the strips of
+        // a row (128 columns, 64 of the one-column sweep) would leave many lanes idle, the flat pair sweep: below 95%
+        // filled for FP32 storage (300x300x80 mixed 18.7 us against 19.9, 130x400x137 19.7 against 26.2; at 98%,
+        // 1000x1000x80 FP32, 184-187 against 177), below 80% for FP64 (101x203x60 8.0 against 9.3, 130x400x137 30.8
+        // against 33.1; at 86%, 387x251x61, 26.0 against 25.2)
+        const int strip = st_size == 4 || ni >= 512 ? 128 : 64;
+        const int filled = (int)(100 * (int64_t)ni / (((int64_t)ni + strip - 1) / strip * strip));
+        if (filled < (st_size == 4 ? 95 : 80))
+            return hdiff_cfg{2, 4, 8, 1};
+        return strip == 128 ? hdiff_cfg{2, 8, 4, 0} : hdiff_cfg{1, 8, 4, 0};
     }
 
     hdiff_cfg hdiff_cfg_for(int st_size, int ct_size, int ni, int nj, int nk) {
@@ -115,9 +123,13 @@ namespace gt355 {
             if (it != g_hdiff.end())
                 c = it->second.cfg;
         }
-        const int impl = tune_param("hdiff_impl", c.impl);
-        if (impl != c.impl)
-            c = impl == 2 ? hdiff_cfg{2, 8, 4, 0} : impl == 1 ? hdiff_cfg{1, 16, 4, 0} : hdiff_cfg{0, 64, 8, 5};
+        // GT355_TUNE_hdiff_impl: 0, 1, 2 (strips) or 3 (the flat pair sweep)
+        const int now = hdiff_is_flat(c) ? 3 : c.impl, impl = tune_param("hdiff_impl", now);
+        if (impl != now)
+            c = impl == 3   ? hdiff_cfg{2, 4, 8, 1}
+                : impl == 2 ? hdiff_cfg{2, 8, 4, 0}
+                : impl == 1 ? hdiff_cfg{1, 16, 4, 0}
+                            : hdiff_cfg{0, 64, 8, 5};
         if (c.impl >= 1) {
             c.a = tune_param("hdiff_jb", c.a);
             c.b = tune_param("hdiff_p", c.b);

@@ -20,11 +20,21 @@ namespace gt355 {
     // Every column-pair sweep shape instantiated for hdiff: X(JB, P).
 #define GT355_HDIFF_SWEEPS2(X) X(4, 4) X(8, 4) X(8, 8) X(16, 4) X(16, 8)
 
+    // Every flat column-pair sweep shape instantiated for hdiff: X(JB, P), none of them among the strips above.
+#define GT355_HDIFF_FLATS(X) X(4, 8)
+
     // One hdiff launch configuration: impl 0 = LDS tile (a, b, c) = (TI, TJ, KC); impl 1 = register sweep
-    // (a, b) = (JB, P); impl 2 = column-pair register sweep (a, b) = (JB, P).
+    // (a, b) = (JB, P); impl 2 = column-pair register sweep (a, b) = (JB, P) over 128-column strips, or with c = 1
+    // over the flat list of pairs.
     struct hdiff_cfg {
         int impl, a, b, c;
     };
+    // whether a configuration is a flat column-pair sweep (c = 1 with any other shape means its strips, as ever)
+    inline bool hdiff_is_flat(const hdiff_cfg &c) {
+#define GT355_IS_FLAT(JB, P) || (c.a == JB && c.b == P)
+        return c.impl == 2 && c.c == 1 && (false GT355_HDIFF_FLATS(GT355_IS_FLAT));
+#undef GT355_IS_FLAT
+    }
 
     // The configuration for an hdiff launch, in this order: environment overrides (GT355_TUNE_hdiff_*), the entry
     // the autotuner recorded for (storage size, compute size, ni, nj, nk), the measured default for the storage type.
