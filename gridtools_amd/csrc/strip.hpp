@@ -2,7 +2,7 @@
 //
 // Used by the single-domain fused kernel (compose.hip) and by the batching form (batch.hip).  The wavefront
 // sweeps k once with ccol/dcol in registers for the first NK levels (the whole column when nk <= NK), as
-// vadv_onchip_kernel does.  At step k it evaluates hdiff at level k+1 for its row in registers:
+// the vertical advection (column.hpp) does.  At step k it evaluates hdiff at level k+1 for its row in registers:
 //   * rows j-2..j+2 of `in` are per-lane loads of the lane's own column;
 //   * the i-1 / i+1 neighbours come from DPP wavefront shifts; lanes 0 and 63 keep the side columns (i0-1 /
 //     i0+64, and i0-2 / i0+65 for the side laplacian), which they load themselves;

@@ -1,0 +1,10 @@
+// Vertical advection, FP32 storage and compute (vadv_launch.hpp).
+#include "vadv_launch.hpp"
+
+namespace gt355 {
+    int vadv_f32(const gt355_field *uts, const gt355_field *us, const gt355_field *wc, const gt355_field *up,
+        const gt355_field *ut, double dtr_stage, int ni, int nj, int nk, hipStream_t stream, void *ext_buf,
+        size_t ext_bytes) {
+        return launch_vadv<float, float>(uts, us, wc, up, ut, dtr_stage, ni, nj, nk, stream, ext_buf, ext_bytes);
+    }
+} // namespace gt355

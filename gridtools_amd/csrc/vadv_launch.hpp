@@ -1,0 +1,322 @@
+// Vertical advection (implicit tridiagonal Thomas solve per column) for gfx950: the kernels and their launch for one
+// storage and compute type, instantiated by vadv_f64.hip, vadv_mixed.hip and vadv_f32.hip.
+//
+// Reference: tests/regression/vertical_advection_dycore.cpp:32-150.  The spec is
+//   multi_pass(execute_forward().k_cached(flush, ccol, dcol).k_cached(fill, u_stage).stage(u_forward...),
+//              execute_backward().k_cached(data_col).stage(u_backward...))
+// and the reference gpu backend fuses both multistages into one launch (stencil/gpu/entry_point.hpp:48-59,
+// 107-124) with one thread per column, u_stage/data_col in register rings (gpu/k_cache.hpp:23-46) and
+// ccol/dcol flushed to HBM temporaries that the backward sweep reads back (gpu/fill_flush.hpp:298-321).
+//
+// Here, too, one lane owns one column and both sweeps run in one launch (column.hpp), with the k-caches in VGPRs and
+// ccol/dcol on chip as far as it holds them: registers, then LDS, then the wavefront's scratch.  Fields that span 4 GiB
+// or more, past the 32-bit buffer offsets, take vadv_scratch_kernel: ccol/dcol in a per-launch scratch buffer in the
+// k-major layout the lanes read coalesced.
+// Results are the functors', operation by operation (built with -ffp-contract=off).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "column.hpp"
+#include "common.hpp"
+#include "functors.hpp"
+
+namespace gt355 {
+    namespace {
+
+        // One column per lane; ccol/dcol of levels 0..nk-2 go to scratch (k-major, column-minor).
+        template <class ST, class CT>
+        __global__ void __launch_bounds__(256) vadv_scratch_kernel(ST *__restrict__ uts_f,
+            const ST *__restrict__ us_f, const ST *__restrict__ wc_f, const ST *__restrict__ up_f,
+            const ST *__restrict__ ut_f, CT dtr, int ni, int nj, int nk, int64_t sj, int64_t sk, int64_t wsj,
+            int64_t wsk, CT *__restrict__ cd_buf, int64_t plane) {
+            const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+            const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
+            if (i >= ni || j >= nj)
+                return;
+            const int64_t col = (int64_t)j * sj + i;
+            const int64_t wcol = (int64_t)j * wsj + i;
+            const int64_t scol = (int64_t)j * ni + i; // scratch column index, plane = ni*nj
+            CT *__restrict__ sc = cd_buf + scol;
+            CT *__restrict__ sd = cd_buf + (int64_t)(nk - 1) * plane + scol;
+
+            // k = 0
+            CT us_c = CT(us_f[col]);
+            CT us_p = CT(us_f[col + sk]);
+            CT w_p_i = CT(wc_f[wcol + wsk]);
+            CT w_p_ip = CT(wc_f[wcol + wsk + 1]);
+            CT up = CT(up_f[col]);
+            fwd_out<CT> r = forward_first<CT>(dtr, w_p_i, w_p_ip, us_c, us_p, up, CT(ut_f[col]), CT(uts_f[col]));
+            sc[0] = r.c;
+            sd[0] = r.d;
+            CT cc_m = r.c, dc_m = r.d;
+#pragma unroll 4
+            for (int k = 1; k < nk - 1; ++k) {
+                const int64_t p = col + (int64_t)k * sk;
+                CT us_m = us_c;
+                us_c = us_p;
+                us_p = CT(us_f[p + sk]);
+                CT w_c_i = w_p_i, w_c_ip = w_p_ip;
+                w_p_i = CT(wc_f[wcol + (int64_t)(k + 1) * wsk]);
+                w_p_ip = CT(wc_f[wcol + (int64_t)(k + 1) * wsk + 1]);
+                up = CT(up_f[p]);
+                r = forward_body<CT>(dtr, w_c_i, w_c_ip, w_p_i, w_p_ip, us_m, us_c, us_p, up, CT(ut_f[p]),
+                    CT(uts_f[p]), cc_m, dc_m, false);
+                sc[(int64_t)k * plane] = r.c;
+                sd[(int64_t)k * plane] = r.d;
+                cc_m = r.c;
+                dc_m = r.d;
+            }
+            // k = nk-1
+            {
+                const int64_t p = col + (int64_t)(nk - 1) * sk;
+                CT us_m = us_c;
+                us_c = us_p;
+                up = CT(up_f[p]);
+                CT dc = forward_last<CT>(
+                    dtr, w_p_i, w_p_ip, us_m, us_c, up, CT(ut_f[p]), CT(uts_f[p]), cc_m, dc_m);
+                // u_backward_function::apply(last_level) (vertical_advection_dycore.cpp:117-121)
+                uts_f[p] = ST(dtr * (dc - up));
+                CT data = dc;
+                // u_backward_function::apply(modify<0,-1>) (vertical_advection_dycore.cpp:110-115)
+#pragma unroll 4
+                for (int k = nk - 2; k >= 0; --k) {
+                    const int64_t q = col + (int64_t)k * sk;
+                    CT cc = sc[(int64_t)k * plane];
+                    CT dd = sd[(int64_t)k * plane];
+                    CT dt = dd - cc * data;
+                    uts_f[q] = ST(dtr * (dt - CT(up_f[q])));
+                    data = dt;
+                }
+            }
+        }
+
+        // The persistent column sweep: WPE wavefronts per SIMD walk the strips (64 columns of one row; the strips of a row
+        // consecutive) with a static stride, so that the wavefronts in flight stay on neighbouring strips.  Each starts
+        // the next strip's first D levels of loads NB levels before the end of a strip's backward sweep, so the next
+        // forward sweep needs no pipeline fill.  Measured against the former kernels (one level bucket per 16 levels,
+        // selects at every level), us: 256x256x80 FP64 37.7 (39.7), mixed 20.4 (21.7); 64x64x80 FP64 12.1 (15.5), mixed
+        // 12.7 (16.3), FP32 10.4 (13.3); 512x512x40 mixed 40.6 (54.2); 192x160x137 FP64 35.1 (124 through memory).
+        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE>
+        __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+        vadv_column_kernel(ST *__restrict__ uts_f, const ST *__restrict__ us_f, const ST *__restrict__ wc_f,
+            const ST *__restrict__ up_f, const ST *__restrict__ ut_f, CT dtr, int ni, int nk, int64_t sj, int64_t sk,
+            int64_t wsj, int64_t wsk, int strips_i, int first, int nitems, int nxcd,
+            CT *scratch, int tail_rows) {
+            __shared__ ST s_up[PARK ? R + TL : 1][64];
+            __shared__ CT s_tail[TL > 0 ? TL * 128 : 1];
+            column_src f{make_rsrc(uts_f), make_rsrc(us_f), make_rsrc(wc_f), make_rsrc(up_f), make_rsrc(ut_f),
+                (uint32_t)(sk * (int64_t)sizeof(ST)), (uint32_t)(wsk * (int64_t)sizeof(ST)), nk};
+            const rsrc_t sc = make_rsrc(scratch + (int64_t)blockIdx.x * tail_rows * 128);
+            // the lane's byte offsets in strip `it` (lanes past ni take column ni-1, computing and storing its bits again)
+            auto offsets = [&](int it, uint32_t &cb, uint32_t &wb) {
+                const int si = it % strips_i, j = it / strips_i;
+                const int i = min(si * 64 + (int)threadIdx.x, ni - 1);
+                cb = (uint32_t)(((int64_t)j * sj + i) * (int64_t)sizeof(ST));
+                wb = (uint32_t)(((int64_t)j * wsj + i) * (int64_t)sizeof(ST));
+            };
+            int it = first + xcd_remap(blockIdx.x, gridDim.x, nxcd);
+            if (it >= nitems)
+                return; // a whole wavefront leaves; there is no barrier in this kernel
+            column_sweep<ST, CT, R, D, TL, NB, PARK, DEEP, MINK> sw;
+            uint32_t cb, wb;
+            offsets(it, cb, wb);
+            sw.prologue(f, cb, wb);
+            for (; it < nitems; it += gridDim.x) {
+                const int nx = it + (int)gridDim.x;
+                uint32_t ncb = cb, nwb = wb;
+                sw.sweep(f, dtr, cb, wb, s_up, s_tail, sc, [&]() {
+                    if (nx < nitems) {
+                        offsets(nx, ncb, nwb);
+                        sw.prologue(f, ncb, nwb);
+                    }
+                });
+                cb = ncb;
+                wb = nwb;
+            }
+        }
+
+        template <class ST, class CT>
+        struct vadv_args {
+            const gt355_field *uts, *us, *wc, *up, *ut;
+            CT dtr;
+            int ni, nj, nk;
+            hipStream_t stream;
+            // scratch: the caller's buffer (ext, budget bytes), or none (budget bytes from the stream's pool)
+            void *ext;
+            size_t budget;
+        };
+
+        // Launches one instantiation: at most WPE wavefronts per SIMD, fewer if the scratch of the levels past R + TL
+        // would exceed the budget, and as many launches as keep each at `rounds` strips per wavefront (0: one launch).
+        // Returns false, launching nothing, if not even a quarter of the wavefronts fit the budget.
+        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE>
+        bool launch_column_as(const vadv_args<ST, CT> &a, int rounds, int *rc) {
+            const int strips_i = (a.ni + 63) / 64;
+            const int64_t items = (int64_t)strips_i * a.nj;
+            if (items >= (int64_t(1) << 31) - (1 << 20))
+                return false;
+            const int tail_rows = DEEP && a.nk > R + TL + 8 ? (a.nk - R - TL - 1) / 8 * 8 : 0;
+            const size_t wave_bytes = (size_t)tail_rows * 128 * sizeof(CT);
+            const int64_t want = std::min<int64_t>(items, (int64_t)cu_count() * 4 * WPE);
+            const int64_t waves = std::min<int64_t>(want, wave_bytes ? (int64_t)(a.budget / wave_bytes) : want);
+            if (waves < 1 || waves * 4 < want)
+                return false;
+            // the pool's buffer is sized for the all-scratch kernel whatever part of it this split uses, so that one
+            // run outside capture readies the stream for captures of every shape that needs no more
+            void *buf = a.ext;
+            *rc = GT355_OK;
+            if (DEEP && !a.ext && (*rc = scratch_for(a.stream, a.budget, &buf)))
+                return true;
+            // launches of equal length
+            const int64_t nlaunch = rounds ? (items + waves * rounds - 1) / (waves * rounds) : 1;
+            const int64_t per = (items + nlaunch - 1) / nlaunch;
+            for (int64_t first = 0; first < items && *rc == GT355_OK; first += per) {
+                const int64_t end = std::min(items, first + per);
+                vadv_column_kernel<ST, CT, R, D, TL, NB, PARK, DEEP, MINK, WPE>
+                    <<<(int)std::min(waves, end - first), 64, 0, a.stream>>>((ST *)a.uts->origin,
+                        (const ST *)a.us->origin, (const ST *)a.wc->origin, (const ST *)a.up->origin,
+                        (const ST *)a.ut->origin, a.dtr, a.ni, a.nk, a.uts->stride[1], a.uts->stride[2],
+                        a.wc->stride[1], a.wc->stride[2], strips_i, (int)first, (int)end, xcd_count(), (CT *)buf,
+                        tail_rows);
+                *rc = check_launch("gt355_vadv");
+            }
+            return true;
+        }
+
+        // Depths that fit registers: an instantiation per number of 8-level blocks below the top one, and per wavefronts
+        // per SIMD and levels of load-ahead where the best of these depends on the number of strips.  Times below in us.
+        template <class ST, class CT, int R, int MINK = R + 1>
+        bool launch_column_blocks(const vadv_args<ST, CT> &a, int *rc) {
+            constexpr bool F32 = sizeof(CT) == 4, S32 = sizeof(ST) == 4;
+            constexpr int NB = R < 32 ? R : 32;
+            // the most wavefronts per SIMD whose registers hold the column and its rings without spills
+            constexpr int WMAX = F32 ? (R <= 32 ? 3 : 2) : R <= (S32 ? 16 : 8) ? 3 : R <= (S32 ? 40 : 32) ? 2 : 1;
+            constexpr int D = !F32 && R <= 32 && R > (S32 ? 24 : 16) ? 4 : 8;
+            const int64_t items = (int64_t)((a.ni + 63) / 64) * a.nj, simds = (int64_t)cu_count() * 4;
+            // Wavefronts per SIMD: a round of w takes about w times a round of one, so the fewest rounds times w, as many
+            // as possible unless fewer save an eighth (400x400x40 FP64, 2.7 strips per SIMD: three rounds of one 50.9, two
+            // of two 59.8; 400x400x40 FP32: one of three 26.2, three of one 29.5; 512x512x16 FP32, 4 strips per SIMD:
+            // two of two 16, two of three 20).
+            auto rounds = [&](int w) { return (items + simds * w - 1) / (simds * w); };
+            int w = WMAX;
+            for (int v = WMAX - 1; v >= 1; --v)
+                if (rounds(v) * v * 8 < rounds(w) * w * 7)
+                    w = v;
+            // A launch per round for large fields: over many rounds in one launch the wavefronts drift apart, and the
+            // memory with them (one launch against one per round: 512x512x80 FP64 161 and 152, 1024x1024x80 744 and 686,
+            // 1536x1536x80 mixed 938 and 824, FP32 925 and 836); smaller or shallower ones lose the wavefronts' overlap at
+            // the rounds' ends (512x512x40 FP64 77.0 and 78.8; 900x900x80 mixed 294 and 307, but 1024x1024x80 356 and 346).
+            const int64_t bytes = items * 64 * a.nk * (int64_t)sizeof(ST);
+            const int per_launch = w < 3 && a.nk >= 32 && bytes >= ((F32 || !S32 ? 150LL : 300LL) << 20) ? 1 : 0;
+            if constexpr (WMAX >= 3)
+                if (w == 3)
+                    return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 3>(a, per_launch, rc);
+            if constexpr (WMAX >= 2)
+                if (w == 2)
+                    return launch_column_as<ST, CT, R, (R >= 40 ? 4 : D), 0, NB, true, false, MINK, 2>(
+                        a, per_launch, rc);
+            // FP32 storage, one wavefront per SIMD: 4 levels ahead keep the reads in flight below what the memory takes
+            // where most SIMDs have one (256x256x80 mixed 20.4 against 22.0 with 8 ahead; 1536x1536x80 in rounds 824 against
+            // 843); 8 levels where few do (64x64x80 12.7 against 13.0) and, a little, over two to four rounds
+            // (512x512x80 79.6 against 80.3, 400x400x80 54.4 against 56.0).  FP64: 8 (64x64x80 12.1 against 14.2).
+            if constexpr (S32 && R >= 40)
+                if (items * 2 > simds && (items <= simds || items > simds * 4))
+                    return launch_column_as<ST, CT, R, 4, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
+            return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
+        }
+
+        template <class ST, class CT>
+        bool launch_column(const vadv_args<ST, CT> &a, int *rc) {
+            const int nk = a.nk;
+#define GT355_COLUMN_BLOCKS(R)                                                                                   \
+    if (nk <= R + 8)                                                                                             \
+        return launch_column_blocks<ST, CT, R>(a, rc)
+            if (nk <= 8)
+                return launch_column_blocks<ST, CT, 8, 2>(a, rc); // the block below the top one is left out at run time
+            GT355_COLUMN_BLOCKS(8);
+            GT355_COLUMN_BLOCKS(16);
+            GT355_COLUMN_BLOCKS(24);
+            GT355_COLUMN_BLOCKS(32);
+            GT355_COLUMN_BLOCKS(40);
+            GT355_COLUMN_BLOCKS(48);
+            GT355_COLUMN_BLOCKS(56);
+            GT355_COLUMN_BLOCKS(64);
+            GT355_COLUMN_BLOCKS(72);
+#undef GT355_COLUMN_BLOCKS
+            // deeper: as many register levels as compile without spills
+#define GT355_DEEP(R, D, TL, NB, PARK)                                                                           \
+    return launch_column_as<ST, CT, R, D, TL, NB, PARK, true, 81, 1>(a, 0, rc)
+            if constexpr (sizeof(CT) == 4) {
+                if (nk <= 112)
+                    GT355_DEEP(104, 8, 0, 32, true);
+                GT355_DEEP(152, 8, 0, 32, true);
+            } else if constexpr (sizeof(ST) == 4) {
+                // u_pos parked while every level fits beside it
+                if (nk <= 112)
+                    GT355_DEEP(96, 8, 8, 32, true);
+                GT355_DEEP(88, 8, 40, 16, false);
+            } else {
+                GT355_DEEP(88, 4, 40, 16, false);
+            }
+#undef GT355_DEEP
+        }
+
+        // ext_buf == nullptr: a path that needs ccol/dcol scratch takes it from the per-stream scratch pool.
+        // Otherwise ext_buf (ext_bytes long) is used and nothing is allocated: the column sweep launches no more
+        // wavefronts than it holds tails for, and vadv_scratch_kernel processes the rows in chunks whose ccol/dcol fit
+        // it (columns are independent, so a chunked launch computes the same bits).
+        template <class ST, class CT>
+        int launch_vadv(const gt355_field *uts, const gt355_field *us, const gt355_field *wc, const gt355_field *up,
+            const gt355_field *ut, double dtr_stage, int ni, int nj, int nk, hipStream_t stream,
+            void *ext_buf = nullptr, size_t ext_bytes = 0) {
+            int64_t sj = uts->stride[1], sk = uts->stride[2];
+            GT355_CHECK(us->stride[1] == sj && us->stride[2] == sk && up->stride[1] == sj && up->stride[2] == sk &&
+                            ut->stride[1] == sj && ut->stride[2] == sk,
+                "gt355_vadv: utens_stage, u_stage, u_pos and utens must share one layout");
+            // the reference keeps dtr_stage as a global_parameter of the storage type (vertical_advection_dycore.cpp:139)
+            const CT dtr_c = CT(ST(dtr_stage));
+            // the column sweep addresses fields through buffer descriptors with 32-bit byte offsets
+            const int64_t span = std::max(((int64_t)(nk - 1) * sk + (int64_t)(nj - 1) * sj + ni) * (int64_t)sizeof(ST),
+                ((int64_t)(nk - 1) * wc->stride[2] + (int64_t)(nj - 1) * wc->stride[1] + ni + 1) * (int64_t)sizeof(ST));
+            const bool fits32 = span < (int64_t(1) << 32);
+            int rc = GT355_OK;
+            if (fits32 && nk <= 80) {
+                GT355_CHECK(nj <= 65535, "gt355_vadv: nj too large");
+                if (launch_column<ST, CT>({uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, nullptr, 0}, &rc))
+                    return rc;
+            }
+            // ccol/dcol of levels 0..nk-2 for every column of a row
+            const size_t row_bytes = sizeof(CT) * (size_t)ni * (size_t)(2 * nk - 1);
+            GT355_CHECK(!ext_buf || row_bytes <= ext_bytes,
+                "gt355_vadv_noalloc: ni = %d, nk = %d needs %zu bytes of ccol/dcol for one row of columns, more "
+                "than the %zu-byte static scratch holds",
+                ni, nk, row_bytes, ext_bytes);
+            int rows = ext_buf ? (int)std::min<size_t>((size_t)nj, ext_bytes / row_bytes) : nj;
+            GT355_CHECK((std::min(rows, nj) + 3) / 4 <= 65535, "gt355_vadv: nj too large");
+            if (fits32 && nk > 80 &&
+                launch_column<ST, CT>({uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, ext_buf,
+                                          ext_buf ? ext_bytes : row_bytes * (size_t)nj},
+                    &rc))
+                return rc;
+            void *buf = ext_buf;
+            if (!ext_buf) {
+                if ((rc = scratch_for(stream, row_bytes * (size_t)nj, &buf)))
+                    return rc;
+            }
+            for (int j0 = 0; j0 < nj; j0 += rows) {
+                const int nr = std::min(rows, nj - j0);
+                dim3 grid((ni + 63) / 64, (nr + 3) / 4);
+                vadv_scratch_kernel<ST, CT><<<grid, 256, 0, stream>>>((ST *)uts->origin + j0 * sj,
+                    (const ST *)us->origin + j0 * sj, (const ST *)wc->origin + j0 * wc->stride[1],
+                    (const ST *)up->origin + j0 * sj, (const ST *)ut->origin + j0 * sj, dtr_c, ni, nr, nk, sj, sk,
+                    wc->stride[1], wc->stride[2], (CT *)buf, (int64_t)ni * nr);
+                if ((rc = check_launch("gt355_vadv")))
+                    return rc;
+            }
+            return GT355_OK;
+        }
+    } // namespace
+} // namespace gt355
