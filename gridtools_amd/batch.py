@@ -69,8 +69,7 @@ class Batch:
 
     def config(self):
         """The launch configuration {form, hjb, hw, w, deep_nk}: the form, the stencil phase's rows per item and
-        workgroups per CU, the persistent grid setting, the depth from which the vertical phase keeps 96 levels in
-        registers."""
+        workgroups per CU, the persistent grid setting, and deep_nk, which no kernel reads any more."""
         c = (ctypes.c_int32 * 5)()
         _abi.call("gt355_batch_get_config", self.handle, c)
         return dict(zip(("form", "hjb", "hw", "w", "deep_nk"), list(c)))

@@ -11,8 +11,8 @@
 //                                                 diffusion in the compute type, not re-read
 // The two-phase form runs the same chain in two persistent launches per timestep, each over every domain: the
 // stencil phase (laplacian and hdiff by the one-column register sweep of sweep.hpp, one wavefront per 64-column x
-// JB-row x level item; lap and u_stage stored) and the vertical phase (the strip sweep of strip.hpp with u_stage read
-// back instead of evaluated).  It evaluates each laplacian once instead of once per row that needs it, at the cost
+// JB-row x level item; lap and u_stage stored) and the vertical phase (batch_vertical.hpp; u_stage read back instead
+// of evaluated).  It evaluates each laplacian once instead of once per row that needs it, at the cost
 // of the u_stage round trip through memory; in the precision form u_stage reaches the vertical phase rounded to
 // FP32 (as in the two-launch composition), where the single-launch forms pass it on in FP64.
 // The k depth is a runtime value (up to 144 levels), so ccol/dcol go to the workgroup's own slot of a scratch
@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "batch_vertical.hpp"
 #include "common.hpp"
 #include "functors.hpp"
 #include "strip.hpp"
@@ -35,14 +36,6 @@ namespace gt355 {
         constexpr int BTI = 64, BTJ = 4, BMAXK = 144;
         // forward steps run up to D-1 levels past a column's top; scratch rows = deepest nk + BPAST
         constexpr int BPAST = 8;
-
-        struct bdom {
-            const void *in, *coeff, *wcon, *u_pos, *utens;
-            void *lap, *u_stage, *utens_stage;
-            int64_t sj, sk;   // shared layout of every field but wcon (origins at grid point (0,0,0))
-            int64_t wsj, wsk; // wcon layout
-            int32_t ni, nj, nk, tiles_i;
-        };
 
         struct bitem {
             int32_t dom, ti, tj, pad;
@@ -220,18 +213,10 @@ namespace gt355 {
         }
 
 
-        // Work item of the strip form: 64 columns (from i0) of row j of one domain; with `flat` set (the two-phase
-        // form's vertical phase), 64 entries of the domain's column list from entry i0 (j unused).
-        struct sitem {
-            int32_t dom, i0, j, flat;
-        };
-        // load-ahead depths of the strip sweep: 4 levels in the single-launch strip form and with 32 register
-        // levels (deeper rings spill there), 8 in the two-phase form's vertical phase, whose kernel then takes 476 of
-        // 512 registers without spills (its one wavefront per SIMD is latency-bound at 4: five loads per level,
-        // 5 MB in flight over the GPU)
-        constexpr int SD = 4, SDV = 8;
+        // load-ahead of the strip sweep: 4 levels (deeper rings spill)
+        constexpr int SD = 4;
         // tail levels a wavefront's scratch holds, for a register part of NK levels
-        constexpr int stail_rows(int nk_reg) { return BMAXK - nk_reg + SDV; }
+        constexpr int stail_rows(int nk_reg) { return BMAXK - nk_reg + 8; }
 
         // The batching form on the strip sweep (strip.hpp): one wavefront per workgroup and per item, no LDS
         // tile, no barrier, ccol/dcol in registers for the first NK levels and in the wavefront's tail scratch
@@ -243,20 +228,11 @@ namespace gt355 {
         //   NK = 32, two wavefronts per SIMD (ccol/dcol of 32 levels fit half the register file): every level
         //   past 32 goes through the tail scratch, but no column runs clamped steps past its top (the batch's
         //   depths start at 40) and two wavefronts hide each other's latency.
-        // The vertical phase with FP32 storage also has a 96-level register part, taken by columns of at least
-        // deep_nk levels: it halves the tail-scratch levels of the deepest columns (ccol/dcol of 96 levels still fit
-        // the register file of one wavefront per SIMD; u_pos of 96 levels in LDS is 24 KiB per wavefront).
-        template <class ST, class CT, int NK, int WPE, bool HD>
+        template <class ST, class CT, int NK, int WPE>
         __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
         batch_strip_kernel(const bdom *__restrict__ doms, const sitem *__restrict__ items, int nitems, CT dtr,
-            CT *__restrict__ scratch, int nxcd, int deep_nk) {
-            constexpr bool DEEP = !HD && NK == 80 && sizeof(ST) == 4;
-            constexpr int KD = !HD && NK == 80 ? SDV : SD;
-            __shared__ ST s_up[DEEP ? 96 : NK][64];
-            // with FP32 storage the 96-level part keeps the first LTAIL tail levels of ccol/dcol in LDS: 24 KiB of
-            // u_pos + 16 KiB of tail per wavefront, the 160 KiB of a CU for its four wavefronts
-            constexpr int LTAIL = DEEP && sizeof(CT) == 8 ? 16 : 0;
-            __shared__ CT s_tail[LTAIL > 0 ? LTAIL * 128 : 1];
+            CT *__restrict__ scratch, int nxcd) {
+            __shared__ ST s_up[NK][64];
             CT *tail = scratch + (int64_t)blockIdx.x * (stail_rows(NK) * 128);
             const int wid = xcd_remap(blockIdx.x, gridDim.x, nxcd);
             for (int it = wid; it < nitems; it += gridDim.x) {
@@ -265,27 +241,8 @@ namespace gt355 {
                 const strip_fields<ST> f{(const ST *)dm.in, (const ST *)dm.coeff, (const ST *)dm.wcon,
                     (const ST *)dm.u_pos, (const ST *)dm.utens, (ST *)dm.u_stage, (ST *)dm.utens_stage,
                     (ST *)dm.lap, dm.sj, dm.sk, dm.sj, dm.sk, dm.sj, dm.sk, dm.sj, dm.sk, dm.wsj, dm.wsk};
-                // the vertical phase takes items of the column list (flagged in the item) or of one row's strip
-                const bool flat = item.flat != 0;
-                if constexpr (!HD && NK == 80) {
-                    // the vertical phase: columns of at most 48 or 64 levels run a register part of that depth
-                    // (a uniform branch per item), not 80 steps with the levels past their top clamped
-                    if (dm.nk <= 48)
-                        hv_strip<ST, CT, 48, KD, true, true, false, HD, !HD>(
-                            f, dtr, dm.ni, dm.nj, dm.nk, item.i0, item.j, s_up, tail, flat);
-                    else if (dm.nk <= 64)
-                        hv_strip<ST, CT, 64, KD, true, true, false, HD, !HD>(
-                            f, dtr, dm.ni, dm.nj, dm.nk, item.i0, item.j, s_up, tail, flat);
-                    else if (DEEP && dm.nk >= deep_nk)
-                        hv_strip<ST, CT, DEEP ? 96 : NK, KD, true, true, true, HD, !HD, LTAIL>(
-                            f, dtr, dm.ni, dm.nj, dm.nk, item.i0, item.j, s_up, tail, flat, s_tail);
-                    else
-                        hv_strip<ST, CT, NK, KD, true, true, true, HD, !HD>(
-                            f, dtr, dm.ni, dm.nj, dm.nk, item.i0, item.j, s_up, tail, flat);
-                } else {
-                    hv_strip<ST, CT, NK, KD, true, true, true, HD, !HD>(
-                        f, dtr, dm.ni, dm.nj, dm.nk, item.i0, item.j, s_up, tail, flat);
-                }
+                hv_strip<ST, CT, NK, SD, true, true, true>(
+                    f, dtr, dm.ni, dm.nj, dm.nk, item.i0, item.j, s_up, tail);
             }
         }
 
@@ -331,7 +288,8 @@ struct gt355_batch {
     int impl;      // 1: 64x4 tiles, ccol/dcol in scratch; 2: 64-column strips, ccol/dcol in registers;
                    // 3: two phases (stencil sweep, then the vertical advection over column-list items)
     int nk_reg;    // strip form: levels of ccol/dcol held in registers (80: one wavefront per SIMD; 32: two)
-    int deep_nk;   // vertical phase, FP32 storage: columns of at least this many levels keep 96 in registers
+    vertical_plan plan; // two-phase form: the vertical items' depth classes
+    int deep_nk;   // a value of the stored configurations that no kernel reads any more
     int ndoms, nitems, dtype, precision, grid, gridmax, cus, rows;
     int w;           // the persistent grid's setting (batch_grid)
     int nhitems[3];  // the stencil phase: items per table
@@ -407,7 +365,7 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
     const int impl_p = form ? form : tune_param("batch_impl", 3);
     const int impl = impl_p == 1 ? 1 : impl_p == 3 ? 3 : 2;
     // register depth of the strip form (GT355_TUNE_batch_nk: 80 or 32)
-    const int nk_reg = tune_param("batch_nk", 80) == 32 ? 32 : 80;
+    const int nk_reg = impl == 2 && tune_param("batch_nk", 80) == 32 ? 32 : 80;
     std::vector<bdom> doms(ndomains);
     std::vector<bitem> items;
     std::vector<sitem> sitems;
@@ -475,15 +433,6 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
                 "gt355_batch_create: domain %d spans 4 GiB or more", d);
             if (!vert) {
                 // a stencil-phase-only domain has no vertical items
-            } else if (impl == 3 && tune_param("batch_flat", 0) != 0) {
-                // the vertical phase on 64 consecutive entries of the domain's column list per item (no partial
-                // strips at row ends; disjoint, so each column has one owner).  Measured slower than row strips on
-                // 64 domains of seed 2024 (2.47 against 2.14 ms per timestep): an item's rows start at any column
-                // and may span two rows, so its requests touch more, unaligned lines
-                GT355_CHECK((int64_t)ni * nj < (int64_t(1) << 31), "gt355_batch_create: domain %d has too many columns",
-                    d);
-                for (int c0 = 0; c0 < ni * nj; c0 += 64)
-                    sitems.push_back(sitem{d, c0, 0, 1});
             } else {
                 const int strips = (ni + 63) / 64;
                 for (int j = 0; j < nj; ++j)
@@ -505,6 +454,9 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
     hipDeviceProp_t p;
     GT355_HIP(hipGetDeviceProperties(&p, current_device()));
     gt355_batch *bt = new gt355_batch{};
+    for (int n = 0; n < VCLASSES; ++n)
+        for (const sitem &s : sitems)
+            bt->plan.end[n] += doms[s.dom].nk > vertical_above(n);
     bt->impl = impl;
     bt->nk_reg = nk_reg;
     bt->ndoms = ndomains;
@@ -546,7 +498,9 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
         maxnk = std::max(maxnk, m.nk);
     bt->rows = maxnk + BPAST;
     const size_t ct = (dt == GT355_F64 || precision == GT355_WIDEN) ? 8 : 4;
-    const size_t per_wg = impl >= 2 ? (size_t)stail_rows(nk_reg) * 128 : 2 * (size_t)bt->rows * 256;
+    const size_t per_wg = impl == 3   ? (size_t)VTAIL_ROWS * 128
+                          : impl == 2 ? (size_t)stail_rows(nk_reg) * 128
+                                      : 2 * (size_t)bt->rows * 256;
     if (e == hipSuccess && bt->gridmax > 0)
         e = hipMalloc(&bt->scratch, ct * per_wg * (size_t)bt->gridmax);
     if (e != hipSuccess) {
@@ -594,30 +548,30 @@ extern "C" int gt355_batch_run(gt355_batch *bt, double dtr_stage, void *stream) 
         }
         if (bt->nitems == 0)
             return GT355_OK; // stencil-phase domains only
-        const int deep_nk = bt->deep_nk;
-#define GT355_BATCH_STRIP(NK, WPE, HD)                                                                          \
+        if (bt->impl == 3) {
+            if (bt->dtype == GT355_F64)
+                batch_vertical_f64(bt->doms, it, bt->plan, bt->grid, dtr_stage, scr, xcd_count(), s);
+            else if (bt->precision == GT355_WIDEN)
+                batch_vertical_mixed(
+                    bt->doms, it, bt->plan, bt->grid, double(float(dtr_stage)), scr, xcd_count(), s);
+            else
+                batch_vertical_f32(bt->doms, it, bt->plan, bt->grid, float(dtr_stage), scr, xcd_count(), s);
+            return check_launch("gt355_batch_run");
+        }
+#define GT355_BATCH_STRIP(NK, WPE)                                                                              \
     if (bt->dtype == GT355_F64)                                                                                 \
-        batch_strip_kernel<double, double, NK, WPE, HD><<<bt->grid, 64, 0, s>>>(bt->doms, it, bt->nitems,          \
-            dtr_stage, (double *)scr, xcd_count(), deep_nk);                                                    \
+        batch_strip_kernel<double, double, NK, WPE><<<bt->grid, 64, 0, s>>>(                                     \
+            bt->doms, it, bt->nitems, dtr_stage, (double *)scr, xcd_count());                                   \
     else if (bt->precision == GT355_WIDEN)                                                                      \
-        batch_strip_kernel<float, double, NK, WPE, HD><<<bt->grid, 64, 0, s>>>(bt->doms, it, bt->nitems,           \
-            double(float(dtr_stage)), (double *)scr, xcd_count(), deep_nk);                                     \
+        batch_strip_kernel<float, double, NK, WPE><<<bt->grid, 64, 0, s>>>(                                      \
+            bt->doms, it, bt->nitems, double(float(dtr_stage)), (double *)scr, xcd_count());                    \
     else                                                                                                        \
-        batch_strip_kernel<float, float, NK, WPE, HD><<<bt->grid, 64, 0, s>>>(bt->doms, it, bt->nitems,            \
-            float(dtr_stage), (float *)scr, xcd_count(), deep_nk);
-        const bool hd = bt->impl == 2;
+        batch_strip_kernel<float, float, NK, WPE><<<bt->grid, 64, 0, s>>>(                                       \
+            bt->doms, it, bt->nitems, float(dtr_stage), (float *)scr, xcd_count());
         if (bt->nk_reg == 32) {
-            if (hd) {
-                GT355_BATCH_STRIP(32, 2, true)
-            } else {
-                GT355_BATCH_STRIP(32, 2, false)
-            }
+            GT355_BATCH_STRIP(32, 2)
         } else {
-            if (hd) {
-                GT355_BATCH_STRIP(80, 1, true)
-            } else {
-                GT355_BATCH_STRIP(80, 1, false)
-            }
+            GT355_BATCH_STRIP(80, 1)
         }
 #undef GT355_BATCH_STRIP
         return check_launch("gt355_batch_run");
@@ -687,26 +641,18 @@ extern "C" int gt355_batch_tune(gt355_batch *bt, int reps, void *stream, int *wg
     GT355_HIP(hipEventCreate(&e1));
     int rc = GT355_OK;
     double best_t = 1e300, t = 0;
-    // the persistent grid of the vertical phase (or of the single-launch forms), then, for FP32 storage, the depth
-    // from which the vertical phase keeps 96 levels in registers
-    const int deep_opts[4] = {81, 89, 97, 1 << 20};
-    const bool deep = bt->impl == 3 && bt->dtype == GT355_F32 && bt->nk_reg == 80;
-    int best_w = bt->w, best_deep = bt->deep_nk;
+    // the persistent grid of the vertical phase (or of the single-launch forms)
+    int best_w = bt->w;
     for (int w = 1; w <= BWG_MAX && rc == GT355_OK; ++w) {
         if (w > 1 && batch_grid(bt, w) == batch_grid(bt, w - 1))
             break; // fewer items than workgroups: larger grids are the same grid
         bt->grid = batch_grid(bt, w);
-        for (int o = 0; o < (deep ? 4 : 1) && rc == GT355_OK; ++o) {
-            if (deep)
-                bt->deep_nk = deep_opts[o];
-            rc = time_runs(bt, reps, s, e0, e1, &t);
-            if (rc == GT355_OK && t < best_t)
-                best_t = t, best_w = w, best_deep = bt->deep_nk;
-        }
+        rc = time_runs(bt, reps, s, e0, e1, &t);
+        if (rc == GT355_OK && t < best_t)
+            best_t = t, best_w = w;
     }
     bt->w = best_w;
     bt->grid = batch_grid(bt, best_w);
-    bt->deep_nk = best_deep;
     // the two-phase form's stencil phase: rows per item and workgroups per CU
     if (bt->impl == 3 && rc == GT355_OK) {
         int best_hjb = bt->hjb, best_hw = bt->hw;

@@ -1,6 +1,6 @@
 // One wavefront's share of the hdiff -> vadv composition: 64 columns of one row j, all levels.
 //
-// Used by the single-domain fused kernel (compose.hip) and by the batching form (batch.hip).  The wavefront
+// Used by the single-domain fused kernel (compose.hip) and by the batching form's strip kernel (batch.hip).  The wavefront
 // sweeps k once with ccol/dcol in registers for the first NK levels (the whole column when nk <= NK), as
 // the vertical advection (column.hpp) does.  At step k it evaluates hdiff at level k+1 for its row in registers:
 //   * rows j-2..j+2 of `in` are per-lane loads of the lane's own column;
@@ -11,8 +11,7 @@
 // forward Thomas step in the compute type.  u_pos is parked in LDS for the backward sweep.
 // TAIL: columns deeper than NK continue in a runtime loop over blocks of D levels whose ccol/dcol go to the
 // wavefront's `tail` scratch (64 lanes x (c, d) per level); the backward sweep reads them back, then finishes the
-// register part.  With TL > 0 the first TL tail levels use the LDS array `s_tail` instead (TL a multiple of D), so
-// that only columns deeper than NK + TL move ccol/dcol through memory.
+// register part.
 // Every load and store is unconditional, with levels clamped to the top (a step above the top recomputes or
 // overwrites the top with the same bits, or with a value the top's own step overwrites later in program order),
 // which keeps the code straight-line and the load counter exact.  Addresses are buffer descriptors plus 32-bit
@@ -52,19 +51,10 @@ namespace gt355 {
     // column must belong to exactly one wavefront.  NARROW: in a strip that ends past ni, lanes past ni take lane
     // ni-1's results and store the same bits to column ni-1 as that lane (ds_bpermute per level); callers pass
     // NARROW = false only when every strip is full (ni a multiple of 64).
-    // HD = false: the vertical advection alone, with u_stage read from memory (written beforehand by the batching
-    // form's stencil phase) instead of evaluated; nothing but utens_stage is stored.
-    // FLAT (with HD = false only): when `flat` is set, the wavefront's columns are 64 consecutive entries of the
-    // domain's column list (column n is i = n % ni of row j = n / ni), starting at i0 (j is not used); lanes past the
-    // last column repeat it, computing and storing the same bits as its own lane.  Columns are independent in the
-    // vertical advection, so no lane idles at the end of a row.
-    template <class ST, class CT, int NK, int D, bool NARROW, bool LAP, bool TAIL, bool HD = true, bool FLAT = false,
-        int TL = 0>
+    template <class ST, class CT, int NK, int D, bool NARROW, bool LAP, bool TAIL>
     __device__ __forceinline__ void hv_strip(const strip_fields<ST> &f, CT dtr, int ni, int nj, int nk, int i0,
-        int j, ST (*s_up)[64], CT *tail, bool flat = false, CT *s_tail = nullptr) {
+        int j, ST (*s_up)[64], CT *tail) {
         static_assert(NK % D == 0, "tail blocks start on a ring-slot boundary");
-        static_assert(TL % D == 0, "LDS tail blocks are whole ring blocks");
-        static_assert(!(FLAT && HD), "the column list form has no horizontal neighbours");
         constexpr int64_t S = sizeof(ST);
         const int lane = threadIdx.x & 63;
         const bool left = lane < 32;
@@ -74,14 +64,7 @@ namespace gt355 {
         const int ic = min(i0 + lane, ni + 1);
         const int e1c = left ? i0 - 1 : min(i0 + 64, ni + 1);
         const int e2c = left ? i0 - 2 : min(i0 + 65, ni + 1);
-        int iv = min(i0 + lane, ni - 1);
-        if constexpr (FLAT) {
-            if (flat) {
-                const int n = min(i0 + lane, ni * nj - 1);
-                j = n / ni;
-                iv = n - j * ni;
-            }
-        }
+        const int iv = min(i0 + lane, ni - 1);
         const int top = nk - 1;
         auto lvl = [&](int L) { return (uint32_t)min(L, top); };
 
@@ -109,8 +92,6 @@ namespace gt355 {
             asm volatile("" : "+s"(csk_b));
             asm volatile("" : "+s"(sk_b));
             asm volatile("" : "+s"(wsk_b));
-            if constexpr (!HD)
-                asm volatile("" : "+s"(osk_b));
         };
 
         // register rings, level L in slot L % D: hdiff inputs of level L (consumed at step L-1), vadv inputs of
@@ -119,11 +100,6 @@ namespace gt355 {
         ST b_uts[D], b_up[D], b_ut[D];
         ST a_wi[D], a_wip[D];
         auto load_h = [&](int L, int s) {
-            if constexpr (!HD) {
-                // u_stage of the lane's column (default cache policy: the stencil phase has just written it)
-                h_c[2][s] = bload<ST>(r_ust, v_o, lvl(L) * osk_b);
-                return;
-            }
             const uint32_t o = lvl(L) * isk_b;
             h_c[0][s] = bload<ST>(r_in, v_c0, o);
             h_c[1][s] = bload<ST>(r_in, v_c1, o);
@@ -143,12 +119,7 @@ namespace gt355 {
             b_ut[s] = bload<ST, CPOL_NT>(r_ut, v_col, o);
         };
         auto load_a = [&](int L, int s) {
-            // wcon at i and i + 1: column i0 + 64 of a strip is the first column of the next strip's line, so the
-            // batch's vertical phase (HD = false) keeps wcon lines in L2 (default policy) for the neighbouring item
-            // on the same XCD; non-temporal loads there fetched those lines twice (vertical-phase reads 5.29 ->
-            // 5.02 GB per timestep, 2.042 -> 1.998 ms)
-            const two<ST> w = HD ? bload2<ST, CPOL_NT>(r_wc, v_wc, lvl(L) * wsk_b)
-                                 : bload2<ST>(r_wc, v_wc, lvl(L) * wsk_b);
+            const two<ST> w = bload2<ST, CPOL_NT>(r_wc, v_wc, lvl(L) * wsk_b);
             a_wi[s] = w.a;
             a_wip[s] = w.b;
         };
@@ -156,8 +127,6 @@ namespace gt355 {
         // hdiff at level L for the lane's column (horizontal_diffusion.cpp:41-46, 56-60, 70-74, 86-90), inputs in
         // slot s; stored as u_stage (and lap), returned in the compute type
         auto hdiff_level = [&](int L, int s) -> CT {
-            if constexpr (!HD)
-                return CT(h_c[2][s]);
             const CT c0 = CT(h_c[0][s]), c1 = CT(h_c[1][s]), c2 = CT(h_c[2][s]), c3 = CT(h_c[3][s]),
                      c4 = CT(h_c[4][s]);
             const CT e1m = CT(h_e1[0][s]), e10 = CT(h_e1[1][s]), e1p = CT(h_e1[2][s]), e2 = CT(h_e2[s]);
@@ -237,20 +206,12 @@ namespace gt355 {
             // memory operations stay at their step; arithmetic may move across steps
             __builtin_amdgcn_sched_barrier(6);
         }
-        // the tail level n (0-based past NK): the LDS tail for n < TL, the scratch tail beyond (a block of D levels
-        // is wholly on one side; a generic pointer serves both)
-        auto tail_at = [&](int n) -> CT * {
-            if constexpr (TL > 0)
-                if (n < TL)
-                    return s_tail + (int64_t)n * 128;
-            return tail + (int64_t)(n - TL) * 128;
-        };
         if constexpr (TAIL) {
             for (int kb = NK; kb < nk; kb += D) {
 #pragma clang loop unroll(full)
                 for (int s = 0; s < D; ++s) {
                     const fwd_out<CT> r = fstep(kb + s, s, (s + 1) % D, false, true);
-                    CT *t = tail_at(kb + s - NK);
+                    CT *t = tail + (int64_t)(kb + s - NK) * 128;
                     t[lane] = r.c;
                     t[64 + lane] = r.d;
                 }
@@ -266,7 +227,7 @@ namespace gt355 {
                 CT rc[D], rd[D], rp[D];
 #pragma clang loop unroll(full)
                 for (int s = 0; s < D; ++s) {
-                    const CT *t = tail_at(kb + s - NK);
+                    const CT *t = tail + (int64_t)(kb + s - NK) * 128;
                     rc[s] = t[lane];
                     rd[s] = t[64 + lane];
                     rp[s] = CT(bload<ST, CPOL_NT>(r_up, v_col, lvl(kb + s) * sk_b));

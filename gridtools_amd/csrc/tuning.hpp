@@ -50,7 +50,7 @@ namespace gt355 {
         int hjb;     // stencil phase: rows per item (8, 16, 32)
         int hw;      // stencil phase: workgroups per CU (2, 4, 8)
         int w;       // vertical phase (or the single-launch forms): the persistent grid's setting (1..4)
-        int deep_nk; // vertical phase, FP32 storage: columns of at least this many levels keep 96 in registers
+        int deep_nk; // stored and returned as ever; the vertical phase chooses its register levels by depth alone
     };
     bool find_batch_cfg(uint64_t sig, int st_size, int ct_size, int impl, batch_cfg *out);
     void record_batch_cfg(uint64_t sig, int st_size, int ct_size, int impl, batch_cfg cfg, double us);

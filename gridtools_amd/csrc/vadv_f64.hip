@@ -1,4 +1,5 @@
-// Vertical advection, FP64 storage and compute (vadv_launch.hpp).
+// Vertical advection, FP64 storage and compute (vadv_launch.hpp), and the batching form's vertical phase (batch_vertical.hpp).
+#include "batch_vertical.hpp"
 #include "vadv_launch.hpp"
 
 namespace gt355 {
@@ -6,5 +7,9 @@ namespace gt355 {
         const gt355_field *ut, double dtr_stage, int ni, int nj, int nk, hipStream_t stream, void *ext_buf,
         size_t ext_bytes) {
         return launch_vadv<double, double>(uts, us, wc, up, ut, dtr_stage, ni, nj, nk, stream, ext_buf, ext_bytes);
+    }
+    void batch_vertical_f64(const bdom *doms, const sitem *items, const vertical_plan &plan, int grid, double dtr,
+        void *scratch, int nxcd, hipStream_t stream) {
+        launch_batch_vertical<double, double>(doms, items, plan, grid, dtr, scratch, nxcd, stream);
     }
 } // namespace gt355

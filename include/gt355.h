@@ -321,8 +321,7 @@ int gt355_graph_destroy(void *graph_exec);
  * domains have the dtype of domains[0].in.  Forms (chosen at create time, GT355_TUNE_batch_impl):
  *   3 (default), two phases: one persistent launch of the laplacian and hdiff register sweep over every domain's
  *     (64-column strip, row block, level) items, then one of the vertical advection over every domain's 64-column
- *     strips of one row (GT355_TUNE_batch_flat=1: 64 consecutive entries of its column list per item instead),
- *     u_stage read back from memory; results equal gt355_laplacian + gt355_hdiff_vadv's two-launch
+ *     strips of one row, u_stage read back from memory; results equal gt355_laplacian + gt355_hdiff_vadv's two-launch
  *     composition bit for bit (in the precision form u_stage reaches the vertical phase rounded to FP32);
  *   2, one launch: strips evaluate hdiff and the vertical advection together, u_stage passed on in the compute
  *     type; results equal gt355_laplacian + the fused gt355_hdiff_vadv bit for bit;
