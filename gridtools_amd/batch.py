@@ -68,8 +68,8 @@ class Batch:
         return w.value, us.value
 
     def config(self):
-        """The launch configuration {form, hjb, hw, w, deep_nk}: the form, the stencil phase's rows per item and
-        workgroups per CU, the persistent grid setting, and deep_nk, which no kernel reads any more."""
+        """The launch configuration {form, hjb, hw, w, deep_nk}: the form, the stencil phase's rows per
+        wavefront (hjb 8, 16 or 32: 1, 2 or 4), the persistent grid setting w; hw and deep_nk choose nothing any more."""
         c = (ctypes.c_int32 * 5)()
         _abi.call("gt355_batch_get_config", self.handle, c)
         return dict(zip(("form", "hjb", "hw", "w", "deep_nk"), list(c)))

@@ -10,8 +10,7 @@
 //   vadv(utens_stage, u_stage, wcon, u_pos, utens) (vertical_advection_dycore.cpp:32-150), u_stage taken from the
 //                                                 diffusion in the compute type, not re-read
 // The two-phase form runs the same chain in two persistent launches per timestep, each over every domain: the
-// stencil phase (laplacian and hdiff by the one-column register sweep of sweep.hpp, one wavefront per 64-column x
-// JB-row x level item; lap and u_stage stored) and the vertical phase (batch_vertical.hpp; u_stage read back instead
+// stencil phase (laplacian and hdiff by the flat column-pair sweep of sweep.hpp; lap and u_stage stored) and the vertical phase (batch_vertical.hpp; u_stage read back instead
 // of evaluated).  It evaluates each laplacian once instead of once per row that needs it, at the cost
 // of the u_stage round trip through memory; in the precision form u_stage reaches the vertical phase rounded to
 // FP32 (as in the two-launch composition), where the single-launch forms pass it on in FP64.
@@ -246,34 +245,77 @@ namespace gt355 {
             }
         }
 
-        // Work item of the two-phase form's stencil phase: columns [i0, i0+64) x rows [j0, j0+JB) of level k.
+        // Work of the two-phase form's stencil phase: `n` (at most HCHUNK) consecutive wavefronts of one domain's flat
+        // column-pair sweep, from wavefront w0.
+        constexpr int HCHUNK = 64;
+        struct hchunk {
+            int32_t dom, w0, n, pad;
+        };
+        // Work item of the stencil phase for domains the flat sweep does not take: columns [i0, i0+64) x rows
+        // [j0, j0+HJB) of level k.
+        constexpr int HJB = 8;
         struct hitem {
             int32_t dom, i0, j0, k;
         };
 
         // The stencil phase: laplacian (stored as lap where the domain has one) and hdiff (stored as u_stage) of every
-        // domain in the phase, one register
-        // sweep per item, items taken by wavefronts with a static stride; the item order (domain, level, row block,
-        // strip) keeps the wavefronts in flight on neighbouring strips, whose rim rows they share through L2.
+        // domain in the phase by the flat column-pair sweep (sweep.hpp), one wavefront per 60 outputs of a domain's list,
+        // the chunks in the order domain, level, row block, pair.  Widths of a batch are ragged, and the flat list fills
+        // its lanes at any width.  What bounds it: the memory, two streams in and two out (it runs at 4.4 TB/s; without
+        // the laplacian's store 239 MB of 955 less and 60 us), then wavefronts in flight: two rows per wavefront (fewer
+        // registers) beat four and eight although more of the rows are read again, from L2.  A table of one entry per
+        // wavefront, as the strips had, is read from memory by every wavefront before its domain's entry and its
+        // rows: chunks of 64 stay in the scalar cache.  16 domains (60 M points), both phases, us: the one-column strips
+        // 529 (FP64 1006), here with one entry per wavefront 517 with four rows, with chunks 507 with two (520 with four,
+        // 531 with eight; FP64 934, 944, 954).
         template <class ST, class CT, int JB, int P>
-        __global__ void __launch_bounds__(256) batch_hdiff_kernel(const bdom *__restrict__ doms,
-            const hitem *__restrict__ items, int nitems, int nxcd) {
-            const int nw = gridDim.x * 4;
-            const int w0 = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x, nxcd) * 4 + (threadIdx.x >> 6));
-            for (int it = w0; it < nitems; it += nw) {
-                const hitem item = items[it];
-                const bdom dm = doms[item.dom];
-                // global-address-space views of the table's pointers (global_* rather than flat_* accesses)
-                const gptr<ST> ust = (gptr<ST>)dm.u_stage, lap = (gptr<ST>)dm.lap;
-                const gptr<const ST> in = (gptr<const ST>)dm.in, co = (gptr<const ST>)dm.coeff;
-                // the laplacian is stored where the domain has a lap field (a uniform branch per item)
-                if (dm.lap)
-                    hdiff_sweep_wave<ST, CT, JB, P, true, gptr<ST>, gptr<const ST>>(ust, in, co, lap, dm.ni, dm.nj,
-                        dm.sj, dm.sk, dm.sj, dm.sk, dm.sj, dm.sk, item.i0, item.j0, item.k);
+        __global__ void __launch_bounds__(256) batch_flat_kernel(
+            const bdom *__restrict__ doms, const hchunk *__restrict__ chunks, int nxcd) {
+            const int n = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x, nxcd) * 4 + (threadIdx.x >> 6));
+            const hchunk c = chunks[n / HCHUNK];
+            if (n % HCHUNK >= c.n)
+                return; // a whole wavefront leaves; there is no barrier in this kernel
+            const int w = c.w0 + n % HCHUNK;
+            const bdom &dm = doms[c.dom];
+            const uint32_t sj = (uint32_t)(dm.sj * (int64_t)sizeof(ST)), sk = (uint32_t)(dm.sk * (int64_t)sizeof(ST));
+            const int np = flat_entries(dm.ni), blocks = (dm.nj + JB - 1) / JB;
+            const hdiff_flat_args g{dm.ni, dm.nj, np, blocks, sj, sk, sj, sk, sj, sk, np * blocks * dm.nk};
+            // `in` is addressed from its lowest read point (-2, -2, 0), so every byte offset is non-negative
+            const rsrc_t r_in = make_rsrc((const ST *)dm.in - 2 - 2 * dm.sj), r_co = make_rsrc(dm.coeff),
+                         r_o = make_rsrc(dm.u_stage);
+            // the laplacian is stored where the domain has a lap field
+            if (dm.lap) {
+                const rsrc_t r_l = make_rsrc(dm.lap);
+                if (dm.ni % 2)
+                    hdiff_flat_wave<ST, CT, JB, P, true, true>(r_o, r_in, r_co, r_l, g, w);
                 else
-                    hdiff_sweep_wave<ST, CT, JB, P, false, gptr<ST>, gptr<const ST>>(ust, in, co, ust, dm.ni, dm.nj,
-                        dm.sj, dm.sk, dm.sj, dm.sk, dm.sj, dm.sk, item.i0, item.j0, item.k);
+                    hdiff_flat_wave<ST, CT, JB, P, true, false>(r_o, r_in, r_co, r_l, g, w);
+            } else {
+                if (dm.ni % 2)
+                    hdiff_flat_wave<ST, CT, JB, P, false, true>(r_o, r_in, r_co, r_o, g, w);
+                else
+                    hdiff_flat_wave<ST, CT, JB, P, false, false>(r_o, r_in, r_co, r_o, g, w);
             }
+        }
+
+        // Domains of one column or fewer rows than the flat sweep's: one register sweep per item (sweep.hpp).
+        template <class ST, class CT>
+        __global__ void __launch_bounds__(256) batch_hdiff_kernel(
+            const bdom *__restrict__ doms, const hitem *__restrict__ items, int nitems) {
+            const int it = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+            if (it >= nitems)
+                return;
+            const hitem item = items[it];
+            const bdom dm = doms[item.dom];
+            // global-address-space views of the table's pointers (global_* rather than flat_* accesses)
+            const gptr<ST> ust = (gptr<ST>)dm.u_stage, lap = (gptr<ST>)dm.lap;
+            const gptr<const ST> in = (gptr<const ST>)dm.in, co = (gptr<const ST>)dm.coeff;
+            if (dm.lap)
+                hdiff_sweep_wave<ST, CT, HJB, 4, true, gptr<ST>, gptr<const ST>>(ust, in, co, lap, dm.ni, dm.nj, dm.sj,
+                    dm.sk, dm.sj, dm.sk, dm.sj, dm.sk, item.i0, item.j0, item.k);
+            else
+                hdiff_sweep_wave<ST, CT, HJB, 4, false, gptr<ST>, gptr<const ST>>(ust, in, co, ust, dm.ni, dm.nj, dm.sj,
+                    dm.sk, dm.sj, dm.sk, dm.sj, dm.sk, item.i0, item.j0, item.k);
         }
     } // namespace
 } // namespace gt355
@@ -283,7 +325,8 @@ using namespace gt355;
 struct gt355_batch {
     bdom *doms;    // device table
     void *items;   // device table: bitem (tile form) or sitem (strip and two-phase forms)
-    void *hitems[3]; // device tables: hitem (the two-phase form's stencil phase) for 8, 16 and 32 rows per item
+    void *hchunks[3]; // device tables: hchunk (the two-phase form's stencil phase) for 1, 2 and 4 rows per wavefront
+    void *hitems[3];  // and, with each, the hitems of the domains that its flat sweep does not take
     void *scratch; // ccol/dcol of every workgroup the grid may have, in the compute type
     int impl;      // 1: 64x4 tiles, ccol/dcol in scratch; 2: 64-column strips, ccol/dcol in registers;
                    // 3: two phases (stencil sweep, then the vertical advection over column-list items)
@@ -292,8 +335,9 @@ struct gt355_batch {
     int deep_nk;   // a value of the stored configurations that no kernel reads any more
     int ndoms, nitems, dtype, precision, grid, gridmax, cus, rows;
     int w;           // the persistent grid's setting (batch_grid)
-    int nhitems[3];  // the stencil phase: items per table
-    int hjb, hw;     // the stencil phase: rows per item, workgroups per CU
+    int nhchunks[3], nhitems[3]; // the stencil phase: entries per table
+    int hjb;         // the stencil phase: 8, 16 or 32 for 1, 2 or 4 rows per wavefront
+    int hw;          // a value of the stored configurations that no launch reads any more
     uint64_t sig;    // signature of the domain list (key of the tuner's table)
 };
 
@@ -306,15 +350,9 @@ namespace gt355 {
         inline int batch_grid(const gt355_batch *bt, int w) {
             return std::min<int>(bt->nitems, bt->cus * (bt->impl >= 2 ? (bt->nk_reg == 32 ? 4 : 2) * w : w));
         }
-        // the stencil phase's tables: index of 8, 16 or 32 rows per item
+        // the stencil phase's tables: index of the hjb settings, and the rows per wavefront each stands for
         inline int hjb_index(int hjb) { return hjb == 8 ? 0 : hjb == 32 ? 2 : 1; }
-        constexpr int HJB_OF[3] = {8, 16, 32};
-        // the stencil phase's grid: four wavefronts per workgroup, hw workgroups per CU (8: one round at 8
-        // wavefronts per SIMD), each wavefront striding through the items
-        inline int stencil_grid(const gt355_batch *bt) {
-            const int64_t n = bt->nhitems[hjb_index(bt->hjb)];
-            return (int)std::max<int64_t>(1, std::min<int64_t>((n + 3) / 4, (int64_t)bt->cus * bt->hw));
-        }
+        constexpr int HJB_OF[3] = {8, 16, 32}, HROWS[3] = {1, 2, 4};
         // FNV-1a over the batch's form, types and domain sizes: the key of its tuned configuration
         inline uint64_t batch_signature(int impl, int dt, int precision, const gt355_batch_domain *d, int n) {
             uint64_t h = 1469598103934665603ULL;
@@ -370,6 +408,7 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
     std::vector<bitem> items;
     std::vector<sitem> sitems;
     std::vector<hitem> hitems[3];
+    std::vector<hchunk> hchunks[3];
     for (int d = 0; d < ndomains; ++d) {
         const gt355_batch_domain &b = domains[d];
         const int ni = b.ni, nj = b.nj, nk = b.nk, ph = b.phases;
@@ -416,14 +455,22 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
         m.nk = nk;
         m.tiles_i = (ni + BTI - 1) / BTI;
         if (impl == 3 && sten) {
-            // the stencil phase's item tables for every row-block height the tuner may choose
+            // the stencil phase's tables for every row-block height the tuner may choose
             for (int h = 0; h < 3; ++h) {
-                const int jb = HJB_OF[h];
-                const int strips = (ni + 63) / 64, rowblocks = (nj + jb - 1) / jb;
+                const int jb = HROWS[h];
+                const int64_t entries = (int64_t)flat_entries(ni) * ((nj + jb - 1) / jb) * nk;
+                if (ni >= 2 && nj >= jb && entries < (int64_t(1) << 31) - 64) {
+                    // the list's first and last entries are rim pairs
+                    const int waves = (int)((entries - 2 + FLAT_OW - 1) / FLAT_OW);
+                    for (int w = 0; w < waves; w += HCHUNK)
+                        hchunks[h].push_back(hchunk{d, w, std::min(HCHUNK, waves - w), 0});
+                    continue;
+                }
+                const int strips = (ni + 63) / 64, rowblocks = (nj + HJB - 1) / HJB;
                 for (int k = 0; k < nk; ++k)
                     for (int rb = 0; rb < rowblocks; ++rb)
                         for (int si = 0; si < strips; ++si)
-                            hitems[h].push_back(hitem{d, si * 64, rb * jb, k});
+                            hitems[h].push_back(hitem{d, si * 64, rb * HJB, k});
             }
         }
         if (impl >= 2) {
@@ -464,8 +511,10 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
     bt->dtype = dt;
     bt->precision = precision;
     bt->cus = p.multiProcessorCount;
-    for (int h = 0; h < 3; ++h)
+    for (int h = 0; h < 3; ++h) {
+        bt->nhchunks[h] = (int)hchunks[h].size();
         bt->nhitems[h] = (int)hitems[h].size();
+    }
     // the launch configuration: the tuner's entry for this list of domains if one was recorded (or loaded), else
     // the measured defaults and the caller's grid setting; environment knobs override both
     bt->sig = batch_signature(impl, dt, precision, domains, ndomains);
@@ -486,11 +535,16 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
         e = hipMemcpy(bt->doms, doms.data(), sizeof(bdom) * doms.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess && item_bytes)
         e = hipMemcpy(bt->items, item_src, item_bytes, hipMemcpyHostToDevice);
+    auto table = [&](void **p, const auto &v) {
+        const size_t bytes = v.size() * sizeof(v[0]);
+        if (e == hipSuccess && bytes)
+            e = hipMalloc(p, bytes);
+        if (e == hipSuccess && bytes)
+            e = hipMemcpy(*p, v.data(), bytes, hipMemcpyHostToDevice);
+    };
     for (int h = 0; h < 3; ++h) {
-        if (e == hipSuccess && !hitems[h].empty())
-            e = hipMalloc(&bt->hitems[h], sizeof(hitem) * hitems[h].size());
-        if (e == hipSuccess && !hitems[h].empty())
-            e = hipMemcpy(bt->hitems[h], hitems[h].data(), sizeof(hitem) * hitems[h].size(), hipMemcpyHostToDevice);
+        table(&bt->hchunks[h], hchunks[h]);
+        table(&bt->hitems[h], hitems[h]);
     }
     // each batch owns its scratch, so batches on different streams never share it
     int maxnk = 0;
@@ -506,8 +560,10 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
     if (e != hipSuccess) {
         (void)hipFree(bt->doms);
         (void)hipFree(bt->items);
-        for (void *h : bt->hitems)
-            (void)hipFree(h);
+        for (int h = 0; h < 3; ++h) {
+            (void)hipFree(bt->hchunks[h]);
+            (void)hipFree(bt->hitems[h]);
+        }
         (void)hipFree(bt->scratch);
         delete bt;
         return hip_fail(e, "gt355_batch_create");
@@ -524,28 +580,32 @@ extern "C" int gt355_batch_run(gt355_batch *bt, double dtr_stage, void *stream) 
     if (bt->impl >= 2) {
         const sitem *it = (const sitem *)bt->items;
         const int hx = hjb_index(bt->hjb);
-        if (bt->impl == 3 && bt->nhitems[hx] > 0) {
-            const hitem *hi = (const hitem *)bt->hitems[hx];
-            const int nh = bt->nhitems[hx], hg = stencil_grid(bt);
-#define GT355_BATCH_HDIFF(JB)                                                                                   \
-    if (bt->dtype == GT355_F64)                                                                                 \
-        batch_hdiff_kernel<double, double, JB, 4><<<hg, 256, 0, s>>>(bt->doms, hi, nh, xcd_count());            \
-    else if (bt->precision == GT355_WIDEN)                                                                      \
-        batch_hdiff_kernel<float, double, JB, 4><<<hg, 256, 0, s>>>(bt->doms, hi, nh, xcd_count());             \
-    else                                                                                                        \
-        batch_hdiff_kernel<float, float, JB, 4><<<hg, 256, 0, s>>>(bt->doms, hi, nh, xcd_count());
-            if (bt->hjb == 8) {
-                GT355_BATCH_HDIFF(8)
-            } else if (bt->hjb == 32) {
-                GT355_BATCH_HDIFF(32)
-            } else {
-                GT355_BATCH_HDIFF(16)
-            }
-#undef GT355_BATCH_HDIFF
+#define GT355_BATCH_STENCIL(ST, CT)                                                                             \
+    {                                                                                                           \
+        const hchunk *hc = (const hchunk *)bt->hchunks[hx];                                                     \
+        const hitem *hi = (const hitem *)bt->hitems[hx];                                                        \
+        const int nc = bt->nhchunks[hx] * (HCHUNK / 4), ni = bt->nhitems[hx];                                   \
+        if (nc && hx == 0)                                                                                      \
+            batch_flat_kernel<ST, CT, 1, 5><<<nc, 256, 0, s>>>(bt->doms, hc, xcd_count());                      \
+        else if (nc && hx == 1)                                                                                 \
+            batch_flat_kernel<ST, CT, 2, 6><<<nc, 256, 0, s>>>(bt->doms, hc, xcd_count());                      \
+        else if (nc)                                                                                            \
+            batch_flat_kernel<ST, CT, 4, 8><<<nc, 256, 0, s>>>(bt->doms, hc, xcd_count());                      \
+        if (ni)                                                                                                 \
+            batch_hdiff_kernel<ST, CT><<<(ni + 3) / 4, 256, 0, s>>>(bt->doms, hi, ni);                          \
+    }
+        if (bt->impl == 3 && bt->nhchunks[hx] + bt->nhitems[hx] > 0) {
+            if (bt->dtype == GT355_F64)
+                GT355_BATCH_STENCIL(double, double)
+            else if (bt->precision == GT355_WIDEN)
+                GT355_BATCH_STENCIL(float, double)
+            else
+                GT355_BATCH_STENCIL(float, float)
             int rc = check_launch("gt355_batch_run");
             if (rc)
                 return rc;
         }
+#undef GT355_BATCH_STENCIL
         if (bt->nitems == 0)
             return GT355_OK; // stencil-phase domains only
         if (bt->impl == 3) {
@@ -595,8 +655,10 @@ extern "C" int gt355_batch_destroy(gt355_batch *bt) {
         return GT355_OK;
     (void)hipFree(bt->doms);
     (void)hipFree(bt->items);
-    for (void *h : bt->hitems)
-        (void)hipFree(h);
+    for (int h = 0; h < 3; ++h) {
+        (void)hipFree(bt->hchunks[h]);
+        (void)hipFree(bt->hitems[h]);
+    }
     (void)hipFree(bt->scratch);
     delete bt;
     return GT355_OK;
@@ -653,20 +715,16 @@ extern "C" int gt355_batch_tune(gt355_batch *bt, int reps, void *stream, int *wg
     }
     bt->w = best_w;
     bt->grid = batch_grid(bt, best_w);
-    // the two-phase form's stencil phase: rows per item and workgroups per CU
+    // the two-phase form's stencil phase: rows per wavefront
     if (bt->impl == 3 && rc == GT355_OK) {
-        int best_hjb = bt->hjb, best_hw = bt->hw;
-        const int hws[3] = {2, 4, 8};
-        for (int h = 0; h < 3 && rc == GT355_OK; ++h)
-            for (int q = 0; q < 3 && rc == GT355_OK; ++q) {
-                bt->hjb = HJB_OF[h];
-                bt->hw = hws[q];
-                rc = time_runs(bt, reps, s, e0, e1, &t);
-                if (rc == GT355_OK && t < best_t)
-                    best_t = t, best_hjb = bt->hjb, best_hw = bt->hw;
-            }
+        int best_hjb = bt->hjb;
+        for (int h = 0; h < 3 && rc == GT355_OK; ++h) {
+            bt->hjb = HJB_OF[h];
+            rc = time_runs(bt, reps, s, e0, e1, &t);
+            if (rc == GT355_OK && t < best_t)
+                best_t = t, best_hjb = bt->hjb;
+        }
         bt->hjb = best_hjb;
-        bt->hw = best_hw;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

@@ -271,7 +271,7 @@ namespace gt355 {
         int total;                             // list entries
     };
     // list entries per row block
-    inline int flat_entries(int ni) { return ((ni + 1) / 2 + 2 + FLAT_ALIGN - 1) / FLAT_ALIGN * FLAT_ALIGN; }
+    __host__ __device__ inline int flat_entries(int ni) { return ((ni + 1) / 2 + 2 + FLAT_ALIGN - 1) / FLAT_ALIGN * FLAT_ALIGN; }
     template <class ST, class CT, int JB, int P, bool LAP, bool ODD>
     __device__ __forceinline__ void hdiff_flat_wave(
         rsrc_t r_out, rsrc_t r_in, rsrc_t r_co, rsrc_t r_lap, const hdiff_flat_args &g, int w) {

@@ -47,8 +47,8 @@ namespace gt355 {
 
     // A batch's launch configuration, as the batch tuner records it for one list of domains (its signature).
     struct batch_cfg {
-        int hjb;     // stencil phase: rows per item (8, 16, 32)
-        int hw;      // stencil phase: workgroups per CU (2, 4, 8)
+        int hjb;     // stencil phase: 8, 16 or 32 for 1, 2 or 4 rows per wavefront
+        int hw;      // stored and returned as ever (2, 4, 8); the stencil phase has one wavefront per piece of work
         int w;       // vertical phase (or the single-launch forms): the persistent grid's setting (1..4)
         int deep_nk; // stored and returned as ever; the vertical phase chooses its register levels by depth alone
     };

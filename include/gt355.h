@@ -319,9 +319,9 @@ int gt355_graph_destroy(void *graph_exec);
  * utens_stage = vadv(utens_stage, u_stage, wcon, u_pos, utens).  Domains: ni, nj >= 1, 2 <= nk <= 144; `in`
  * readable on [-2, n+2) in i and j, wcon on [0, ni+1) in i; every field but wcon shares the layout of `in`.  All
  * domains have the dtype of domains[0].in.  Forms (chosen at create time, GT355_TUNE_batch_impl):
- *   3 (default), two phases: one persistent launch of the laplacian and hdiff register sweep over every domain's
- *     (64-column strip, row block, level) items, then one of the vertical advection over every domain's 64-column
- *     strips of one row, u_stage read back from memory; results equal gt355_laplacian + gt355_hdiff_vadv's two-launch
+ *   3 (default), two phases: one launch of the laplacian and hdiff register sweep over every domain's
+ *     (level, row block, column pair) list, then one persistent launch of the vertical advection over every domain's
+ *     64-column strips of one row, u_stage read back from memory; results equal gt355_laplacian + gt355_hdiff_vadv's two-launch
  *     composition bit for bit (in the precision form u_stage reaches the vertical phase rounded to FP32);
  *   2, one launch: strips evaluate hdiff and the vertical advection together, u_stage passed on in the compute
  *     type; results equal gt355_laplacian + the fused gt355_hdiff_vadv bit for bit;
