@@ -271,7 +271,8 @@ namespace gt355 {
         template <class ST, class CT, int JB, int P>
         __global__ void __launch_bounds__(256) batch_flat_kernel(
             const bdom *__restrict__ doms, const hchunk *__restrict__ chunks, int nxcd) {
-            const int n = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x, nxcd) * 4 + (threadIdx.x >> 6));
+            const int n = __builtin_amdgcn_readfirstlane(
+                xcd_remap_groups(blockIdx.x, gridDim.x, nxcd, XCD_GROUP) * 4 + (threadIdx.x >> 6));
             const hchunk c = chunks[n / HCHUNK];
             if (n % HCHUNK >= c.n)
                 return; // a whole wavefront leaves; there is no barrier in this kernel

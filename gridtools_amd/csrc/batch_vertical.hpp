@@ -104,7 +104,7 @@ namespace gt355 {
             // u_pos of R + TL levels and ccol/dcol of TL levels, at most a quarter of the CU's LDS
             __shared__ __attribute__((aligned(16))) char lds[40 << 10];
             const rsrc_t sc = make_rsrc(scratch + (int64_t)blockIdx.x * (VTAIL_ROWS * 128));
-            int it = xcd_remap(blockIdx.x, gridDim.x, nxcd);
+            int it = xcd_remap_groups(blockIdx.x, gridDim.x, nxcd, XCD_GROUP);
 #define GT355_VCLASS(N, ...) vertical_class<ST, CT, __VA_ARGS__>(doms, items, plan.end[N], it, dtr, lds, sc)
             if constexpr (F32) {
                 GT355_VCLASS(0, 136, 8, 0, 32, true, false, 113);

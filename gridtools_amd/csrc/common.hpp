@@ -101,6 +101,24 @@ namespace gt355 {
         return (n % nxcd) * per + n / nxcd;
     }
 
+    // The same in groups: each XCD takes `group` consecutive logical ids in turn, so neighbours still share an L2 but
+    // all XCDs move through memory together instead of in eighths of it.  For streams past the caches, where the
+    // distance between the XCDs' accesses costs memory efficiency (hdiff FP64 512x512x80 94.8 us in eighths, 87.5 in
+    // groups of 16, 90.1 in groups of 1, 92.4 in groups of 256; 300x700x90 89.4, 80.3, 82.5, 85.7); fields that the
+    // Infinity Cache holds lose a little at the groups' ends (FP32 512x512x80 39.9 and 40.7).  Not for the
+    // vertical advection, whose wavefronts stay at their strips for a whole column (1536x1536x80 mixed 816 and 857).
+    // group = 0: xcd_remap.  Ids beyond the largest multiple of nxcd * group keep their natural position.
+    constexpr int XCD_GROUP = 16;
+    __device__ __forceinline__ int xcd_remap_groups(int n, int total, int nxcd, int group) {
+        if (group == 0)
+            return xcd_remap(n, total, nxcd);
+        const int span = nxcd * group, full = total / span * span;
+        if (n >= full || nxcd <= 1)
+            return n;
+        const int slot = n / nxcd;
+        return (slot / group * nxcd + n % nxcd) * group + slot % group;
+    }
+
     // Buffer-resource access: a field is a buffer descriptor (base in scalar registers), a level is a uniform
     // 32-bit byte offset (soffset) and a lane's column a 32-bit byte offset (voffset).  One level offset serves
     // every field of one layout, so a load costs no per-lane or per-field address arithmetic.  Offsets are byte

@@ -137,9 +137,10 @@ namespace gt355 {
         template <class ST, class CT, int JB, int P>
         __global__ void __launch_bounds__(256) hdiff_sweep_kernel(ST *__restrict__ out, const ST *__restrict__ in,
             const ST *__restrict__ coeff, int ni, int nj, int nk, int64_t osj, int64_t osk, int64_t isj, int64_t isk,
-            int64_t csj, int64_t csk, int strips_i, int strips_j, int nblocks, int nxcd) {
+            int64_t csj, int64_t csk, int strips_i, int strips_j, int nblocks, int nxcd, int group) {
             // wave-uniform by construction; readfirstlane tells the compiler, so the side columns become scalar loads
-            const int wid = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, nblocks, nxcd) * 4 + (threadIdx.x >> 6));
+            const int wid = __builtin_amdgcn_readfirstlane(
+                xcd_remap_groups(blockIdx.x, nblocks, nxcd, group) * 4 + (threadIdx.x >> 6));
             const int total = strips_i * strips_j * nk;
             if (wid >= total)
                 return; // a whole wavefront leaves; there is no barrier in this kernel
@@ -156,8 +157,9 @@ namespace gt355 {
         template <class ST, class CT, int JB, int P>
         __global__ void __launch_bounds__(256) hdiff_sweep2_kernel(ST *__restrict__ out, const ST *__restrict__ in,
             const ST *__restrict__ coeff, int ni, int nj, int nk, int64_t osj, int64_t osk, int64_t isj, int64_t isk,
-            int64_t csj, int64_t csk, int strips_i, int strips_j, int nblocks, int nxcd) {
-            const int wid = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, nblocks, nxcd) * 4 + (threadIdx.x >> 6));
+            int64_t csj, int64_t csk, int strips_i, int strips_j, int nblocks, int nxcd, int group) {
+            const int wid = __builtin_amdgcn_readfirstlane(
+                xcd_remap_groups(blockIdx.x, nblocks, nxcd, group) * 4 + (threadIdx.x >> 6));
             const int total = strips_i * strips_j * nk;
             if (wid >= total)
                 return; // a whole wavefront leaves; there is no barrier in this kernel
@@ -172,8 +174,10 @@ namespace gt355 {
         // (sweep.hpp: hdiff_flat_wave).
         template <class ST, class CT, int JB, int P, bool ODD>
         __global__ void __launch_bounds__(256) hdiff_flat_kernel(ST *__restrict__ out, const ST *__restrict__ in,
-            const ST *__restrict__ coeff, hdiff_flat_args g, int waves, int nblocks, int nxcd) {
-            const int w = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, nblocks, nxcd) * 4 + (threadIdx.x >> 6));
+            const ST *__restrict__ coeff, hdiff_flat_args g, int waves, int nblocks, int nxcd,
+            int group) {
+            const int w = __builtin_amdgcn_readfirstlane(
+                xcd_remap_groups(blockIdx.x, nblocks, nxcd, group) * 4 + (threadIdx.x >> 6));
             if (w >= waves)
                 return; // a whole wavefront leaves; there is no barrier in this kernel
             const rsrc_t r_out = make_rsrc(out);
@@ -208,6 +212,14 @@ namespace gt355 {
             return check_launch("gt355_hdiff");
         }
 
+        // The sweeps' XCD mapping: groups where the three fields take at least `mib` MiB.  The strips from 256 MiB, past
+        // the Infinity Cache (1536x1536x80 mixed 402 us in eighths, 389 in groups; 1000x1000x60 136 and 132); the flat
+        // pair sweep from 32 MiB (387x251x61 mixed 16.5 and 16.2, 300x300x80 18.9 and 18.0; 101x203x60, 15 MiB, 5.9
+        // and 6.0).
+        int hdiff_group(int ni, int nj, int nk, size_t es, int64_t mib) {
+            return 3 * (int64_t)ni * nj * nk * (int64_t)es >= mib << 20 ? XCD_GROUP : 0;
+        }
+
         template <class ST, class CT, int JB, int P>
         int launch_hdiff_sweep(const gt355_field *out, const gt355_field *in, const gt355_field *coeff, int ni,
             int nj, int nk, hipStream_t stream) {
@@ -218,7 +230,7 @@ namespace gt355 {
             hdiff_sweep_kernel<ST, CT, JB, P><<<(int)blocks, 256, 0, stream>>>((ST *)out->origin,
                 (const ST *)in->origin, (const ST *)coeff->origin, ni, nj, nk, out->stride[1], out->stride[2],
                 in->stride[1], in->stride[2], coeff->stride[1], coeff->stride[2], strips_i, strips_j, (int)blocks,
-                xcd_count());
+                xcd_count(), hdiff_group(ni, nj, nk, sizeof(ST), 256));
             return check_launch("gt355_hdiff");
         }
 
@@ -265,12 +277,13 @@ namespace gt355 {
             const int waves = (g.total - 2 + FLAT_OW - 1) / FLAT_OW, blocks = (waves + 3) / 4;
             // `in` is addressed from its lowest read point (-2, -2, 0), so every byte offset is non-negative
             const ST *in0 = (const ST *)in->origin - 2 - 2 * in->stride[1];
+            const int group = hdiff_group(ni, nj, nk, sizeof(ST), 32);
             if (ni % 2)
                 hdiff_flat_kernel<ST, CT, JB, P, true><<<blocks, 256, 0, stream>>>(
-                    (ST *)out->origin, in0, (const ST *)coeff->origin, g, waves, blocks, xcd_count());
+                    (ST *)out->origin, in0, (const ST *)coeff->origin, g, waves, blocks, xcd_count(), group);
             else
                 hdiff_flat_kernel<ST, CT, JB, P, false><<<blocks, 256, 0, stream>>>(
-                    (ST *)out->origin, in0, (const ST *)coeff->origin, g, waves, blocks, xcd_count());
+                    (ST *)out->origin, in0, (const ST *)coeff->origin, g, waves, blocks, xcd_count(), group);
             return check_launch("gt355_hdiff");
         }
 
@@ -289,7 +302,7 @@ namespace gt355 {
             hdiff_sweep2_kernel<ST, CT, JB, P><<<(int)blocks, 256, 0, stream>>>((ST *)out->origin,
                 (const ST *)in->origin, (const ST *)coeff->origin, ni, nj, nk, out->stride[1], out->stride[2],
                 in->stride[1], in->stride[2], coeff->stride[1], coeff->stride[2], strips_i, strips_j, (int)blocks,
-                xcd_count());
+                xcd_count(), hdiff_group(ni, nj, nk, sizeof(ST), 256));
             return check_launch("gt355_hdiff");
         }
 

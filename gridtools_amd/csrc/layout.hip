@@ -187,7 +187,7 @@ namespace gt355 {
             typedef W vecb __attribute__((ext_vector_type(VB)));
             const int ld = ta | 1;
             constexpr int UN = VA == 1 ? 8 : 4;
-            const int t = xcd_remap(blockIdx.x, ntiles, nxcd);
+            const int t = xcd_remap_groups(blockIdx.x, ntiles, nxcd, NT ? XCD_GROUP : 0);
             const uint32_t it_a = (uint32_t)t % tiles_a, r = (uint32_t)t / tiles_a, it_b = r % tiles_b;
             int64_t so, dof;
             outer_offsets<uint32_t>(d, r / tiles_b, so, dof);
@@ -319,7 +319,8 @@ namespace gt355 {
                         };
                         const bool va = side(src, d.ss, d.a, ta, na), vb = side(dst, d.ds, d.b, tb, nb);
                         // whole lines of arrays past what the Infinity Cache would keep for the next call are streams
-                        // (301x303x137 FP64 86 -> 73 us non-temporal, 256x256x80 35.9 -> 37.5)
+                        // (301x303x137 FP64 86 -> 73 us non-temporal, 256x256x80 35.9 -> 37.5), and their tiles go to the XCDs in
+                        // groups (512x512x80 FP64 135 -> 128 us, FP32 75 -> 73; 197x261x73 FP64, not one, 28.5 -> 30.0)
                         const bool nt = (int64_t)sizeof(W) * na * nb * outer >= (int64_t(64) << 20);
                         auto magic = [](int n) { return n == 1 ? 0u : (uint32_t)(((uint64_t(1) << 32) + n - 1) / n); };
                         if (ntiles <= (int64_t(1) << 23)) { // one workgroup per tile
