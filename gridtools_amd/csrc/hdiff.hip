@@ -291,10 +291,11 @@ namespace gt355 {
         int launch_hdiff_sweep2(const gt355_field *out, const gt355_field *in, const gt355_field *coeff, int ni,
             int nj, int nk, hipStream_t stream) {
             // an odd ni or unaligned rows: FP32 storage takes the flat pair sweep (387x251x61 mixed 16.5 us against 19.6
-            // for the one-column sweep), FP64 the one-column sweep (25.2 against 26.0)
+            // for the one-column sweep), FP64 the one-column sweep (25.2 against 26.0), in at least 8 rows (1000x1000x80 316
+            // against 324 in 4)
             if (!pairs_ok(out, in, coeff, ni, sizeof(ST)))
                 return sizeof(ST) == 4 ? launch_hdiff_flat<ST, CT, 4, 8>(out, in, coeff, ni, nj, nk, stream)
-                                       : launch_hdiff_sweep<ST, CT, JB, P>(out, in, coeff, ni, nj, nk, stream);
+                                       : launch_hdiff_sweep<ST, CT, (JB < 8 ? 8 : JB), P>(out, in, coeff, ni, nj, nk, stream);
             int strips_i = (ni + 127) / 128, strips_j = (nj + JB - 1) / JB;
             int64_t waves = (int64_t)strips_i * strips_j * nk;
             int64_t blocks = (waves + 3) / 4;
@@ -509,7 +510,7 @@ extern "C" int gt355_tune_hdiff(int precision, const gt355_field *out, const gt3
             }
             best_of[ci] = std::min(best_of[ci], 1e3 * ms / reps);
         }
-    const hdiff_cfg dflt = hdiff_default_cfg(st, ni);
+    const hdiff_cfg dflt = hdiff_default_cfg(st, ni, nj, nk);
     double dflt_us = 1e30;
     for (size_t ci = 0; ci < cands.size(); ++ci) {
         const hdiff_cfg &c = cands[ci];

@@ -100,23 +100,36 @@ namespace gt355 {
         read_knobs_locked();
     }
 
-    hdiff_cfg hdiff_default_cfg(int st_size, int ni) {
-        // measured defaults (MI355X, autotuner winners at x80 levels): FP32 storage takes the column-pair sweep with
-        // 8-row strips (256x256: 13.5 us, 512x512: 41 us); FP64 storage the one-column sweep with 8-row strips at
-        // 256x256 (22.2 us) and the column-pair sweep from 512 columns on (88 us against 97 us).  Where the strips of
-        // a row (128 columns, 64 of the one-column sweep) would leave many lanes idle, the flat pair sweep: below 95%
-        // filled for FP32 storage (300x300x80 mixed 18.7 us against 19.9, 130x400x137 19.7 against 26.2; at 98%,
-        // 1000x1000x80 FP32, 184-187 against 177), below 80% for FP64 (101x203x60 8.0 against 9.3, 130x400x137 30.8
-        // against 33.1; at 86%, 387x251x61, 26.0 against 25.2)
-        const int strip = st_size == 4 || ni >= 512 ? 128 : 64;
+    hdiff_cfg hdiff_default_cfg(int st_size, int ni, int nj, int nk) {
+        // Measured defaults (MI355X, us), by the storage type, the bytes of the three fields and how well strips fill a
+        // row (128 columns, 64 of the one-column sweep).
+        const int64_t mib = 3 * (int64_t)ni * nj * nk * st_size >> 20;
+        // Small domains are bound by the wavefronts in flight: the flat pair sweep, which splits them finest (128x128x80
+        // mixed 5.97 against 7.31 of the strips, 128x256x80 9.08 and 10.04), two rows per wavefront for FP64 (128x128x80
+        // 7.85 against 8.40, 64x128x80 5.38 and 6.15; 101x203x60 the same 8.06; past 36 MiB 150x150x100 12.3 and 11.9)
+        if (mib < 36)
+            return st_size == 4 ? hdiff_cfg{2, 4, 8, 1} : hdiff_cfg{2, 2, 6, 1};
+        // FP64 past the caches: pairs, 4 rows (512x512x80 82.2 against 87.2 of 8 rows, 300x700x90 76.7 against 79.8 of the
+        // one-column sweep, 1000x1000x80 307 and 315; 384x384x80, 270 MiB, 47.5 and 46.9)
+        if (st_size == 8 && mib >= 400)
+            return hdiff_cfg{2, 4, 4, 0};
+        // Where many lanes of the strips would idle, the flat pair sweep: below 95% filled for FP32 storage (300x300x80
+        // mixed 18.0 against 19.9, 130x400x137 19.7 against 26.2; at 98%, 1000x1000x80 FP32, 184-187 against 177), below
+        // 80% for FP64 (130x400x137 30.8 against 33.1; at 86%, 387x251x61, 26.0 against 25.2)
+        const int strip = st_size == 4 || (ni >= 512 && mib >= 128) ? 128 : 64;
         const int filled = (int)(100 * (int64_t)ni / (((int64_t)ni + strip - 1) / strip * strip));
         if (filled < (st_size == 4 ? 95 : 80))
             return hdiff_cfg{2, 4, 8, 1};
-        return strip == 128 ? hdiff_cfg{2, 8, 4, 0} : hdiff_cfg{1, 8, 4, 0};
+        // FP32 storage: pairs, 8 rows (256x256x80 FP32 12.9, 512x512x80 39.7; 1536x1536x80 mixed 382 against 394 of 16
+        // rows and 445 of 4).  FP64: one column per lane, 4 rows up to 128 MiB (256x256x80 21.8 against 22.3 of 8 rows,
+        // 512x256x40 22.0 against 23.8 of the pairs; 384x384x80 48.4 and 46.9)
+        if (st_size == 4)
+            return hdiff_cfg{2, 8, 4, 0};
+        return mib < 128 ? hdiff_cfg{1, 4, 4, 0} : strip == 128 ? hdiff_cfg{2, 8, 4, 0} : hdiff_cfg{1, 8, 4, 0};
     }
 
     hdiff_cfg hdiff_cfg_for(int st_size, int ct_size, int ni, int nj, int nk) {
-        hdiff_cfg c = hdiff_default_cfg(st_size, ni);
+        hdiff_cfg c = hdiff_default_cfg(st_size, ni, nj, nk);
         {
             std::lock_guard<std::mutex> lock(g_tune_mutex);
             auto it = g_hdiff.find(tune_key{st_size, ct_size, ni, nj, nk});

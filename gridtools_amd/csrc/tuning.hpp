@@ -21,7 +21,7 @@ namespace gt355 {
 #define GT355_HDIFF_SWEEPS2(X) X(4, 4) X(8, 4) X(8, 8) X(16, 4) X(16, 8)
 
     // Every flat column-pair sweep shape instantiated for hdiff: X(JB, P), none of them among the strips above.
-#define GT355_HDIFF_FLATS(X) X(4, 8)
+#define GT355_HDIFF_FLATS(X) X(4, 8) X(2, 6)
 
     // One hdiff launch configuration: impl 0 = LDS tile (a, b, c) = (TI, TJ, KC); impl 1 = register sweep
     // (a, b) = (JB, P); impl 2 = column-pair register sweep (a, b) = (JB, P) over 128-column strips, or with c = 1
@@ -39,8 +39,8 @@ namespace gt355 {
     // The configuration for an hdiff launch, in this order: environment overrides (GT355_TUNE_hdiff_*), the entry
     // the autotuner recorded for (storage size, compute size, ni, nj, nk), the measured default for the storage type.
     hdiff_cfg hdiff_cfg_for(int st_size, int ct_size, int ni, int nj, int nk);
-    // the measured default configuration for a storage size and domain width (no tuned entry, no knob)
-    hdiff_cfg hdiff_default_cfg(int st_size, int ni);
+    // the measured default configuration for a storage size and domain (no tuned entry, no knob)
+    hdiff_cfg hdiff_default_cfg(int st_size, int ni, int nj, int nk);
     // whether a configuration is one of the instantiated ones (hdiff.hip)
     bool hdiff_cfg_instantiated(hdiff_cfg cfg);
     void record_hdiff_cfg(int st_size, int ct_size, int ni, int nj, int nk, hdiff_cfg cfg, double us);

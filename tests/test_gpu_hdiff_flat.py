@@ -30,6 +30,25 @@ def _run(gt, oracle, ni, nj, nk, dtype, precision, mode, shift=0):
     assert not full.any()
 
 
+@pytest.mark.parametrize("jb,p", [(4, 8), (2, 6)])
+@pytest.mark.parametrize("ni,nj,nk", SIZES + [(119, 2, 3), (120, 3, 2), (64, 5, 4)])
+@pytest.mark.parametrize("dtype,precision,mode", FORMS)
+def test_sizes_by_rows(gpu, oracle, monkeypatch, jb, p, ni, nj, nk, dtype, precision, mode):
+    """Four and two rows per wavefront, with the fewest rows each takes and one less."""
+    monkeypatch.setenv("GT355_TUNE_hdiff_impl", "3")
+    monkeypatch.setenv("GT355_TUNE_hdiff_jb", str(jb))
+    monkeypatch.setenv("GT355_TUNE_hdiff_p", str(p))
+    _run(gpu, oracle, ni, nj, nk, dtype, precision, mode)
+
+
+# the sizes around each line of the default rule: 36, 128 (512 columns) and 400 MiB of FP64 fields
+@pytest.mark.parametrize("ni,nj,nk", [(128, 150, 80), (130, 152, 80), (512, 200, 50), (513, 250, 44), (512, 270, 41),
+                                      (640, 400, 69), (301, 700, 84)])
+@pytest.mark.parametrize("dtype,precision,mode", FORMS)
+def test_default_rule_by_size(gpu, oracle, ni, nj, nk, dtype, precision, mode):
+    _run(gpu, oracle, ni, nj, nk, dtype, precision, mode)
+
+
 @pytest.mark.parametrize("ni,nj,nk", SIZES)
 @pytest.mark.parametrize("dtype,precision,mode", FORMS)
 def test_sizes(gpu, oracle, monkeypatch, ni, nj, nk, dtype, precision, mode):
