@@ -176,4 +176,6 @@ def check(rc: int, what: str = "") -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args), name)
+    rc = getattr(_lib or lib(), name)(*args)
+    if rc != 0:
+        check(rc, name)

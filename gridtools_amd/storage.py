@@ -92,13 +92,16 @@ class DataStore:
         slice ``extra``, with the allocation box as bounds -- the SID after core::shift_origin
         (stencil/core/backend.hpp:28-34).  The structure is built once per (origin, extra) and shared: treat it as
         read-only (a launch's host cost is mostly building these)."""
-        o = self.halos if origin is None else tuple(origin)
-        key = (o, tuple(extra))
-        cache = self.__dict__.setdefault("_sids", {})
-        f = cache.get(key)
-        if f is None:
-            f = cache[key] = self._make_sid(o, extra)
-        return f
+        if origin is None:
+            origin = self.halos
+        try:
+            return self._sids[origin, extra]
+        except (AttributeError, KeyError, TypeError):  # not built yet, or given as lists
+            key = (tuple(origin), tuple(extra))
+            cache = self.__dict__.setdefault("_sids", {})
+            if key not in cache:
+                cache[key] = self._make_sid(*key)
+            return cache[key]
 
     def _make_sid(self, o, extra):
         f = _abi.Field()
