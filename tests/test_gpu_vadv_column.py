@@ -1,6 +1,7 @@
 """Vertical advection of columns up to 80 levels: every number of 8-level blocks, at the depths where a block fills or
 overflows by one level, and the strip counts (64 columns each) that change the wavefronts per SIMD, the load-ahead or
-the number of launches.  FP64 and the native FP32 and mixed forms equal the oracle bit for bit, so the tolerance is
+the number of launches; and the two wavefronts per strip that few strips take from 33 to 144 levels, at every number of
+blocks.  FP64 and the native FP32 and mixed forms equal the oracle bit for bit, so the tolerance is
 zero."""
 import numpy as np
 import pytest
@@ -30,3 +31,11 @@ def test_strips_per_simd(gpu, oracle, nj, nk, dtype, precision, mode):
                           (7777, 80, np.float32, 1, "mixed")])
 def test_launch_per_round(gpu, oracle, nj, nk, dtype, precision, mode):
     _check(gpu, oracle, 65, nj, nk, dtype, precision, mode)
+
+
+# 512 strips, the most that run on two wavefronts each on 256 CUs, and 513; partial strips; the block edges
+@pytest.mark.parametrize("ni,nj", [(1, 1), (70, 3), (64, 512), (65, 256), (64, 513)])
+@pytest.mark.parametrize("nk", [32, 33, 48, 81, 103, 104, 105, 112, 113, 136, 144, 145])
+@pytest.mark.parametrize("dtype,precision,mode", FORMS)
+def test_two_wavefronts_per_strip(gpu, oracle, ni, nj, nk, dtype, precision, mode):
+    _check(gpu, oracle, ni, nj, nk, dtype, precision, mode)
