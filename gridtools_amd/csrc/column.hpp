@@ -51,8 +51,11 @@ namespace gt355 {
     }
 
     // The levels below the top block are R in registers, then TL in LDS, then scratch.  MINK: the smallest depth; one that
-    // ends in the block after the R + TL levels, R + TL < nk <= R + TL + 8, is the only one unless DEEP.
-    template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK = R + TL + 1>
+    // ends in the block after the R + TL levels, R + TL < nk <= R + TL + 8, is the only one unless DEEP.  CPOL_W: the cache
+    // policy of wcon, whose column-64 line a strip shares with its neighbour: the default policy keeps it in L2 for a
+    // neighbour that runs later, the non-temporal one leaves the Infinity Cache to other fields.
+    template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK = R + TL + 1,
+        int CPOL_W = 0>
     struct column_sweep {
         static constexpr int BLK = 8;
         static constexpr bool EXIT = MINK <= R + TL;
@@ -77,8 +80,7 @@ namespace gt355 {
         __device__ __forceinline__ void load_a(
             const column_src &f, int s, uint32_t cb, uint32_t wb, uint32_t o, uint32_t ow) {
             a_us[s] = bload<ST, CPOL_NT>(f.us, cb, o);
-            // default policy: the neighbouring strip reads the column-64 line of this one from L2
-            const two<ST> w = bload2<ST>(f.wc, wb, ow);
+            const two<ST> w = bload2<ST, CPOL_W>(f.wc, wb, ow);
             a_wi[s] = w.a;
             a_wip[s] = w.b;
         }

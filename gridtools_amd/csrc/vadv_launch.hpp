@@ -100,7 +100,7 @@ namespace gt355 {
         // forward sweep needs no pipeline fill.  Measured against the former kernels (one level bucket per 16 levels,
         // selects at every level), us: 256x256x80 FP64 37.7 (39.7), mixed 20.4 (21.7); 64x64x80 FP64 12.1 (15.5), mixed
         // 12.7 (16.3), FP32 10.4 (13.3); 512x512x40 mixed 40.6 (54.2); 192x160x137 FP64 35.1 (124 through memory).
-        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE>
+        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE, int CPOL_W>
         __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
         vadv_column_kernel(ST *__restrict__ uts_f, const ST *__restrict__ us_f, const ST *__restrict__ wc_f,
             const ST *__restrict__ up_f, const ST *__restrict__ ut_f, CT dtr, int ni, int nk, int64_t sj, int64_t sk,
@@ -121,7 +121,7 @@ namespace gt355 {
             int it = first + xcd_remap(blockIdx.x, gridDim.x, nxcd);
             if (it >= nitems)
                 return; // a whole wavefront leaves; there is no barrier in this kernel
-            column_sweep<ST, CT, R, D, TL, NB, PARK, DEEP, MINK> sw;
+            column_sweep<ST, CT, R, D, TL, NB, PARK, DEEP, MINK, CPOL_W> sw;
             uint32_t cb, wb;
             offsets(it, cb, wb);
             sw.prologue(f, cb, wb);
@@ -177,7 +177,8 @@ namespace gt355 {
         // Launches one instantiation: at most WPE wavefronts per SIMD, fewer if the scratch of the levels past R + TL
         // would exceed the budget, and as many launches as keep each at `rounds` strips per wavefront (0: one launch).
         // Returns false, launching nothing, if not even a quarter of the wavefronts fit the budget.
-        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE>
+        template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE,
+            int CPOL_W = 0>
         bool launch_column_as(const vadv_args<ST, CT> &a, int rounds, int *rc) {
             const int strips_i = (a.ni + 63) / 64;
             const int64_t items = (int64_t)strips_i * a.nj;
@@ -200,7 +201,7 @@ namespace gt355 {
             const int64_t per = (items + nlaunch - 1) / nlaunch;
             for (int64_t first = 0; first < items && *rc == GT355_OK; first += per) {
                 const int64_t end = std::min(items, first + per);
-                vadv_column_kernel<ST, CT, R, D, TL, NB, PARK, DEEP, MINK, WPE>
+                vadv_column_kernel<ST, CT, R, D, TL, NB, PARK, DEEP, MINK, WPE, CPOL_W>
                     <<<(int)std::min(waves, end - first), 64, 0, a.stream>>>((ST *)a.uts->origin,
                         (const ST *)a.us->origin, (const ST *)a.wc->origin, (const ST *)a.up->origin,
                         (const ST *)a.ut->origin, a.dtr, a.ni, a.nk, a.uts->stride[1], a.uts->stride[2],
@@ -250,6 +251,12 @@ namespace gt355 {
             if constexpr (S32 && R >= 40)
                 if (items * 2 > simds && (items <= simds || items > simds * 4))
                     return launch_column_as<ST, CT, R, 4, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
+            // FP64, all strips at once: the neighbours' lines are shared in flight, so wcon need not stay in the caches,
+            // where other stencils' fields do (hdiff and this in turn, 256x256x80: 65.7 per pair with the default policy,
+            // 60.4 non-temporal, each alone 22 and 38; several rounds: 512x512x80 153.9 and 155.3)
+            if constexpr (!S32 && R >= 40)
+                if (items <= simds)
+                    return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 1, CPOL_NT>(a, 0, rc);
             return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
         }
 
