@@ -121,11 +121,9 @@ namespace gt355 {
         if (filled < (st_size == 4 ? 95 : 80))
             return hdiff_cfg{2, 4, 8, 1};
         // FP32 storage: pairs, 8 rows (256x256x80 FP32 12.9, 512x512x80 39.7; 1536x1536x80 mixed 382 against 394 of 16
-        // rows and 445 of 4).  FP64: one column per lane, 4 rows up to 128 MiB (256x256x80 21.8 against 22.3 of 8 rows,
-        // 512x256x40 22.0 against 23.8 of the pairs; 384x384x80 48.4 and 46.9)
-        if (st_size == 4)
-            return hdiff_cfg{2, 8, 4, 0};
-        return mib < 128 ? hdiff_cfg{1, 4, 4, 0} : strip == 128 ? hdiff_cfg{2, 8, 4, 0} : hdiff_cfg{1, 8, 4, 0};
+        // rows and 445 of 4).  FP64: one column per lane, 8 rows (256x256x80 22.3, 4 rows 22.1 but 26 in a program's first
+        // few hundred launches; 512x256x40 22.1 against 23.9 of the pairs, taken from 512 columns and 128 MiB)
+        return strip == 128 ? hdiff_cfg{2, 8, 4, 0} : hdiff_cfg{1, 8, 4, 0};
     }
 
     hdiff_cfg hdiff_cfg_for(int st_size, int ct_size, int ni, int nj, int nk) {
