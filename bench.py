@@ -825,7 +825,7 @@ def main():
 
     value = P / (ms_per_step * 1e-3)
     dom = va64
-    traffic = measured_traffic("vadv_onchip_kernel<double,double,80")
+    traffic = measured_traffic("vadv_column_kernel<double,double,72")
     line = {
         "metric": "gridpoint-updates/s + % HBM roofline, hdiff & vadv FP64 vs FP32 @256x256x80",
         "value": round(value, 1),

@@ -261,13 +261,14 @@ namespace gt355 {
         // The stencil phase: laplacian (stored as lap where the domain has one) and hdiff (stored as u_stage) of every
         // domain in the phase by the flat column-pair sweep (sweep.hpp), one wavefront per 60 outputs of a domain's list,
         // the chunks in the order domain, level, row block, pair.  Widths of a batch are ragged, and the flat list fills
-        // its lanes at any width.  What bounds it: the memory, two streams in and two out (it runs at 4.4 TB/s; without
-        // the laplacian's store 239 MB of 955 less and 60 us), then wavefronts in flight: two rows per wavefront (fewer
+        // its lanes at any width.  What bounds it: the memory, two streams in and two out (without the laplacian's
+        // store 239 MB of 955 less and 60 us), then wavefronts in flight: two rows per wavefront (fewer
         // registers) beat four and eight although more of the rows are read again, from L2.  A table of one entry per
         // wavefront, as the strips had, is read from memory by every wavefront before its domain's entry and its
         // rows: chunks of 64 stay in the scalar cache.  16 domains (60 M points), both phases, us: the one-column strips
         // 529 (FP64 1006), here with one entry per wavefront 517 with four rows, with chunks 507 with two (520 with four,
-        // 531 with eight; FP64 934, 944, 954).
+        // 531 with eight; FP64 934, 944, 954), and with the XCDs taking groups in turn 476 (FP64 901): the phase in 195 us,
+        // 4.9 TB/s.
         template <class ST, class CT, int JB, int P>
         __global__ void __launch_bounds__(256) batch_flat_kernel(
             const bdom *__restrict__ doms, const hchunk *__restrict__ chunks, int nxcd) {

@@ -93,7 +93,7 @@ namespace gt355 {
         // other in the code, each a loop over its items with the loads of the next item started in the sweep before, so
         // a wavefront fills its pipeline once per class.  Measured against one sweep of 80 clamped steps with the levels past
         // them through scratch (16 domains of 48..384 x 48..384 x 40..137 points, 60 M in all): FP32 storage, FP64
-        // compute 338 -> 290 us, 5.4 TB/s of the 1.56 GB it moves (a tenth more than the fields' bytes: partial strips
+        // compute 338 -> 282 us, 5.5 TB/s of the 1.56 GB it moves (a tenth more than the fields' bytes: partial strips
         // and the wcon line shared by neighbours).  Bound by the memory; a launch per round of strips was slower (6
         // domains 356 us against 343 for both phases), 4 levels of load-ahead about the same (533 against 529).
         template <class ST, class CT>

@@ -255,7 +255,7 @@ namespace gt355 {
     // request only needs element alignment).
     // What bounds it: ~28 vector instructions per point against ~78 of the one-column sweep (mixed form), so requests:
     // a wavefront's rows start anywhere, five lines where an aligned 128-column strip has four.  Full strips therefore
-    // stay with hdiff_pair_wave (512x512x80 FP64 95 us against 93-100 here, 1536x1536x80 mixed 403 against 418-450)
+    // stay with hdiff_pair_wave (512x512x80 FP64 82 us against 85 here, 1536x1536x80 mixed 382 against 394)
     // and ragged widths come here (mixed, us, strips / flat: 387x251x61 19.6 / 16.2, 130x400x137 26.2 / 19.7,
     // 101x203x60 8.3 / 5.9).  All JB + 4 = 8 rows are loaded ahead: one memory latency per wavefront.
     // Rows: block b covers output rows b*JB.., moved up to end at nj (j0 = min(b*JB, nj - JB), nj >= JB); rows that the
