@@ -18,11 +18,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "column.hpp"
-#include "column_duo.hpp"
 #include "common.hpp"
 #include "functors.hpp"
+#include "vadv_duo.hpp"
 
 namespace gt355 {
     namespace {
@@ -139,30 +140,6 @@ namespace gt355 {
             }
         }
 
-        // Two wavefronts per strip (column_duo.hpp), one strip per workgroup.
-        template <class ST, class CT, int NBLK>
-        __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1)))
-        vadv_duo_kernel(ST *__restrict__ uts_f, const ST *__restrict__ us_f, const ST *__restrict__ wc_f,
-            const ST *__restrict__ up_f, const ST *__restrict__ ut_f, CT dtr, int ni, int nk, int64_t sj, int64_t sk,
-            int64_t wsj, int64_t wsk, int strips_i, int nxcd) {
-            using duo = column_duo<ST, CT, NBLK>;
-            __shared__ typename duo::shared sh;
-            const int it = xcd_remap(blockIdx.x, gridDim.x, nxcd);
-            const int lane = threadIdx.x & 63;
-            // (wave-uniform: the two roles are branches, not masks)
-            if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) {
-                const int si = it % strips_i, j = it / strips_i;
-                // lanes past ni take column ni-1, computing and storing its bits again
-                const int i = min(si * 64 + lane, ni - 1);
-                const column_src f{make_rsrc(uts_f), make_rsrc(us_f), make_rsrc(wc_f), make_rsrc(up_f),
-                    make_rsrc(ut_f), (uint32_t)(sk * (int64_t)sizeof(ST)), (uint32_t)(wsk * (int64_t)sizeof(ST)), nk};
-                duo::coefficients(f, dtr, (uint32_t)(((int64_t)j * sj + i) * (int64_t)sizeof(ST)),
-                    (uint32_t)(((int64_t)j * wsj + i) * (int64_t)sizeof(ST)), sh, lane);
-            } else {
-                duo::recurrence(nk, dtr, sh, lane);
-            }
-        }
-
         template <class ST, class CT>
         struct vadv_args {
             const gt355_field *uts, *us, *wc, *up, *ut;
@@ -260,17 +237,6 @@ namespace gt355 {
             return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
         }
 
-        // Depths of 33 to 144 levels, few strips: one instantiation per number of 8-level blocks.
-        template <class ST, class CT, int NBLK>
-        int launch_duo(const vadv_args<ST, CT> &a) {
-            const int strips_i = (a.ni + 63) / 64;
-            vadv_duo_kernel<ST, CT, NBLK><<<strips_i * a.nj, 128, 0, a.stream>>>((ST *)a.uts->origin,
-                (const ST *)a.us->origin, (const ST *)a.wc->origin, (const ST *)a.up->origin,
-                (const ST *)a.ut->origin, a.dtr, a.ni, a.nk, a.uts->stride[1], a.uts->stride[2], a.wc->stride[1],
-                a.wc->stride[2], strips_i, xcd_count());
-            return check_launch("gt355_vadv");
-        }
-
         template <class ST, class CT>
         bool launch_column(const vadv_args<ST, CT> &a, int *rc) {
             const int nk = a.nk;
@@ -284,16 +250,10 @@ namespace gt355 {
                 void *buf;
                 if (nk > 80 && !a.ext && (*rc = scratch_for(a.stream, a.budget, &buf)))
                     return true;
-                switch ((nk + 7) / 8) {
-#define GT355_DUO(N)                                                                                            \
-    case N:                                                                                                     \
-        *rc = launch_duo<ST, CT, N>(a);                                                                         \
-        return true;
-                    GT355_DUO(5) GT355_DUO(6) GT355_DUO(7) GT355_DUO(8) GT355_DUO(9) GT355_DUO(10) GT355_DUO(11)
-                    GT355_DUO(12) GT355_DUO(13) GT355_DUO(14) GT355_DUO(15) GT355_DUO(16) GT355_DUO(17)
-                    GT355_DUO(18)
-#undef GT355_DUO
-                }
+                constexpr auto duo = std::is_same_v<ST, CT> ? (sizeof(CT) == 8 ? vadv_duo_f64 : vadv_duo_f32)
+                                                            : vadv_duo_mixed;
+                *rc = duo(a.uts, a.us, a.wc, a.up, a.ut, a.dtr, a.ni, a.nj, nk, a.stream);
+                return true;
             }
 #define GT355_COLUMN_BLOCKS(R)                                                                                   \
     if (nk <= R + 8)                                                                                             \
