@@ -6,6 +6,7 @@
 // persist the table as text, one entry per line:
 //   hdiff <storage bytes> <compute bytes> <ni> <nj> <nk> <impl> <a> <b> <c> <microseconds>
 //   batch <signature, hex> <storage bytes> <compute bytes> <form> <hjb> <hw> <w> <deep_nk> <microseconds>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -128,22 +129,28 @@ namespace gt355 {
 
     hdiff_cfg hdiff_cfg_for(int st_size, int ct_size, int ni, int nj, int nk) {
         hdiff_cfg c = hdiff_default_cfg(st_size, ni, nj, nk);
+        bool tuned = false;
         {
             std::lock_guard<std::mutex> lock(g_tune_mutex);
             auto it = g_hdiff.find(tune_key{st_size, ct_size, ni, nj, nk});
-            if (it != g_hdiff.end())
+            if ((tuned = it != g_hdiff.end()))
                 c = it->second.cfg;
         }
-        // GT355_TUNE_hdiff_impl: 0, 1, 2 (strips) or 3 (the flat pair sweep)
-        const int now = hdiff_is_flat(c) ? 3 : c.impl, impl = tune_param("hdiff_impl", now);
-        if (impl != now)
+        // GT355_TUNE_hdiff_impl: 0, 1, 2 (strips) or 3 (the flat pair sweep).  It and hdiff_jb / hdiff_p are laid over a
+        // tuned entry of the strips or over one strip shape per width, not over the default rule's shapes: a flat sweep's
+        // rows and loads ahead go with no others, and what a knob names must not depend on the fields' bytes.
+        const int unset = INT_MIN, impl = tune_param("hdiff_impl", unset), jb = tune_param("hdiff_jb", unset),
+                  p = tune_param("hdiff_p", unset);
+        if ((impl != unset || jb != unset || p != unset) && (!tuned || hdiff_is_flat(c)))
+            c = st_size == 4 || ni >= 512 ? hdiff_cfg{2, 8, 4, 0} : hdiff_cfg{1, 8, 4, 0};
+        if (impl != unset && impl != c.impl)
             c = impl == 3   ? hdiff_cfg{2, 4, 8, 1}
                 : impl == 2 ? hdiff_cfg{2, 8, 4, 0}
                 : impl == 1 ? hdiff_cfg{1, 16, 4, 0}
                             : hdiff_cfg{0, 64, 8, 5};
         if (c.impl >= 1) {
-            c.a = tune_param("hdiff_jb", c.a);
-            c.b = tune_param("hdiff_p", c.b);
+            c.a = jb != unset ? jb : c.a;
+            c.b = p != unset ? p : c.b;
         } else {
             c.a = tune_param("hdiff_ti", c.a);
             c.b = tune_param("hdiff_tj", c.b);
