@@ -53,8 +53,10 @@ namespace gt355 {
     int debug_sync_after(const char *what);
     // Marks the calling thread as capturing a graph (gt355_graph_begin .. gt355_graph_end).
     void set_capturing(bool on);
-    // The deep-column scratch buffer of (current device, stream), grown to at least `bytes` (pools.hip).
-    int scratch_for(hipStream_t stream, size_t bytes, void **out);
+    // The deep-column scratch buffer of (current device, stream), of *have bytes: grown to at least `bytes`, except while
+    // the stream is captured.  `shape` orders the calls: one that is captured must not exceed the largest `shape` asked
+    // for outside capture (GT355_EUNSUP), but may find fewer than `bytes` (pools.hip).
+    int scratch_for(hipStream_t stream, size_t bytes, size_t shape, void **out, size_t *have);
     // Frees the pools and retired buffers (gt355_finalize).
     void release_pools();
     // Resolves, on the current device, the device address of gt355_vadv_noalloc's static scratch (vadv.hip).

@@ -9,12 +9,15 @@
 // * Scratch of the deep-column vertical advection: one growing buffer per (device, stream).  A buffer that is
 //   outgrown is retired, not freed: queued work or a captured graph may still use it.  Retired buffers are freed by
 //   gt355_finalize.  Growth during stream capture is refused (a graph must not depend on an allocation made inside
-//   it); run the largest shape once outside capture first.
+//   it); run the largest shape once outside capture first.  A shape ranks by the ccol/dcol of all its columns, and the
+//   buffer holds what the launches need, often a small part of that: a shape that was captured without having run
+//   itself works with what is there.
 // * Debug launch mode: with GT355_DEBUG_SYNC=1 in the environment (or gt355_debug_sync(1)) every launch is followed
 //   by a device synchronisation that reports a failing kernel at its own call, as the reference's debug builds do
 //   (common/cuda_util.hpp:89-93).  It is skipped while the calling thread captures a graph through gt355_graph_begin.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <memory>
 #include <cstdlib>
@@ -63,7 +66,7 @@ namespace gt355 {
             int dev;
             hipStream_t stream;
             void *p;
-            size_t bytes;
+            size_t bytes, shape;
         };
         std::mutex g_scratch_mutex;
         std::vector<scratch_buf> g_scratch;
@@ -108,38 +111,44 @@ namespace gt355 {
 
     void set_capturing(bool on) { t_capturing = on ? 1 : 0; }
 
-    int scratch_for(hipStream_t stream, size_t bytes, void **out) {
+    int scratch_for(hipStream_t stream, size_t bytes, size_t shape, void **out, size_t *have) {
         const int dev = current_device();
         std::lock_guard<std::mutex> lock(g_scratch_mutex);
         scratch_buf *b = nullptr;
         for (auto &s : g_scratch)
             if (s.dev == dev && s.stream == stream)
                 b = &s;
-        if (b && b->bytes >= bytes) {
-            *out = b->p;
-            return GT355_OK;
+        if (!b || b->shape < shape || b->bytes < bytes) {
+            if (stream_capturing(stream)) {
+                if (!b || b->shape < shape) {
+                    set_error("scratch: %zu bytes are needed while the stream is being captured; run the call once "
+                              "with its largest shape outside capture first",
+                        shape);
+                    return GT355_EUNSUP;
+                }
+            } else {
+                if (!b || b->bytes < bytes) {
+                    void *p = nullptr;
+                    hipError_t e = hipMalloc(&p, bytes);
+                    if (e != hipSuccess) {
+                        set_error("scratch: hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+                        return GT355_ENOMEM;
+                    }
+                    if (b) {
+                        // queued launches or a captured graph may still use the old buffer: keep it until gt355_finalize
+                        g_retired.push_back(b->p);
+                        b->p = p;
+                        b->bytes = bytes;
+                    } else {
+                        g_scratch.push_back(scratch_buf{dev, stream, p, bytes, 0});
+                        b = &g_scratch.back();
+                    }
+                }
+                b->shape = std::max(b->shape, shape);
+            }
         }
-        if (stream_capturing(stream)) {
-            set_error("scratch: %zu bytes are needed while the stream is being captured; run the call once with "
-                      "its largest shape outside capture first",
-                bytes);
-            return GT355_EUNSUP;
-        }
-        void *p = nullptr;
-        hipError_t e = hipMalloc(&p, bytes);
-        if (e != hipSuccess) {
-            set_error("scratch: hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-            return GT355_ENOMEM;
-        }
-        if (b) {
-            // queued launches or a captured graph may still use the old buffer: keep it until gt355_finalize
-            g_retired.push_back(b->p);
-            b->p = p;
-            b->bytes = bytes;
-        } else {
-            g_scratch.push_back(scratch_buf{dev, stream, p, bytes});
-        }
-        *out = p;
+        *out = b->p;
+        *have = b->bytes;
         return GT355_OK;
     }
 

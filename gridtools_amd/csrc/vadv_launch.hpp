@@ -146,14 +146,27 @@ namespace gt355 {
             CT dtr;
             int ni, nj, nk;
             hipStream_t stream;
-            // scratch: the caller's buffer (ext, budget bytes), or none (budget bytes from the stream's pool)
+            // scratch: the caller's buffer of ext_bytes, or the stream's pool; shape: ccol/dcol of all columns (nk > 80)
             void *ext;
-            size_t budget;
+            size_t ext_bytes, shape;
         };
 
+        // The pool's buffer for launches that use `bytes` of it.  Never less than 64 MiB or, if that is less, the shape's
+        // ccol/dcol: the launches of any shape of no more ccol/dcol then fit a buffer that it finds while it is captured,
+        // in fewer wavefronts or in chunks of rows.
+        template <class ST, class CT>
+        int pool_scratch(const vadv_args<ST, CT> &a, size_t bytes, void **buf, size_t *have) {
+            return scratch_for(a.stream, std::max(bytes, std::min(a.shape, size_t(64) << 20)), a.shape, buf, have);
+        }
+
         // Launches one instantiation: at most WPE wavefronts per SIMD, fewer if the scratch of the levels past R + TL
-        // would exceed the budget, and as many launches as keep each at `rounds` strips per wavefront (0: one launch).
-        // Returns false, launching nothing, if not even a quarter of the wavefronts fit the budget.
+        // would exceed the caller's buffer or, of the pool, 256 MiB and the shape's ccol/dcol, and as many launches as keep
+        // each at `rounds` strips per wavefront (0: one launch).  Returns false, launching nothing, if not even a quarter of
+        // the wavefronts fit.  Where under half the lanes have a column the time is the rounds', not the memory's, and
+        // vadv_scratch_kernel, which runs all strips at once, takes those that would need more rounds for lack of scratch (us,
+        // wavefronts as the shape's ccol/dcol hold / all / vadv_scratch_kernel: FP64 3x4096x300 859 / 519 / 564, FP32
+        // 2x4096x300 938 / 319 / 323) and, over several rounds, those with half as many levels again in scratch as on chip
+        // (FP64 16x4096x300 542 against 526, 400 levels 788 and 707; FP32 320 and 319, 474 and 430).
         template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE,
             int CPOL_W = 0>
         bool launch_column_as(const vadv_args<ST, CT> &a, int rounds, int *rc) {
@@ -164,15 +177,22 @@ namespace gt355 {
             const int tail_rows = DEEP && a.nk > R + TL + 8 ? (a.nk - R - TL - 1) / 8 * 8 : 0;
             const size_t wave_bytes = (size_t)tail_rows * 128 * sizeof(CT);
             const int64_t want = std::min<int64_t>(items, (int64_t)cu_count() * 4 * WPE);
-            const int64_t waves = std::min<int64_t>(want, wave_bytes ? (int64_t)(a.budget / wave_bytes) : want);
-            if (waves < 1 || waves * 4 < want)
-                return false;
-            // the pool's buffer is sized for the all-scratch kernel whatever part of it this split uses, so that one
-            // run outside capture readies the stream for captures of every shape that needs no more
+            auto fit = [&](size_t bytes) -> int64_t {
+                const int64_t n = wave_bytes ? std::min<int64_t>(want, (int64_t)(bytes / wave_bytes)) : want;
+                const bool few_lanes = a.ni < strips_i * 32, deep = tail_rows * 2 >= (R + TL + 8) * 3;
+                return n * 4 < want || (few_lanes && (n < want || (deep && want < items))) ? 0 : n;
+            };
             void *buf = a.ext;
+            int64_t waves = fit(a.ext ? a.ext_bytes : std::max(a.shape, size_t(256) << 20));
             *rc = GT355_OK;
-            if (DEEP && !a.ext && (*rc = scratch_for(a.stream, a.budget, &buf)))
-                return true;
+            if (DEEP && waves && !a.ext) {
+                size_t have = 0;
+                if ((*rc = pool_scratch(a, waves * wave_bytes, &buf, &have)))
+                    return true;
+                waves = fit(have);
+            }
+            if (waves < 1)
+                return false;
             // launches of equal length
             const int64_t nlaunch = rounds ? (items + waves * rounds - 1) / (waves * rounds) : 1;
             const int64_t per = (items + nlaunch - 1) / nlaunch;
@@ -245,10 +265,11 @@ namespace gt355 {
             // 31.9; mixed 256x128x80 14.3 and 12.7, 128x128x137 24.4 and 19.6; FP32 256x128x80 14.2 and 11.6.  20 levels
             // FP64 256x128 6.4 and 6.9; 640 strips, 256x160x80 FP64, 27.2 and 31.9).
             if (nk > 32 && nk <= 144 && (int64_t)((a.ni + 63) / 64) * a.nj * 2 <= (int64_t)cu_count() * 4) {
-                // (past 80 levels the pool's buffer is asked for as by the other kernels, so that what a capture refuses
-                // does not depend on the domain's size)
+                // (past 80 levels the pool is asked as by the other kernels, so that what a capture refuses does not
+                // depend on the domain's size)
                 void *buf;
-                if (nk > 80 && !a.ext && (*rc = scratch_for(a.stream, a.budget, &buf)))
+                size_t have;
+                if (nk > 80 && !a.ext && (*rc = pool_scratch(a, 0, &buf, &have)))
                     return true;
                 constexpr auto duo = std::is_same_v<ST, CT> ? (sizeof(CT) == 8 ? vadv_duo_f64 : vadv_duo_f32)
                                                             : vadv_duo_mixed;
@@ -309,7 +330,7 @@ namespace gt355 {
             int rc = GT355_OK;
             if (fits32 && nk <= 80) {
                 GT355_CHECK(nj <= 65535, "gt355_vadv: nj too large");
-                if (launch_column<ST, CT>({uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, nullptr, 0}, &rc))
+                if (launch_column<ST, CT>({uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, nullptr, 0, 0}, &rc))
                     return rc;
             }
             // ccol/dcol of levels 0..nk-2 for every column of a row
@@ -321,14 +342,23 @@ namespace gt355 {
             int rows = ext_buf ? (int)std::min<size_t>((size_t)nj, ext_bytes / row_bytes) : nj;
             GT355_CHECK((std::min(rows, nj) + 3) / 4 <= 65535, "gt355_vadv: nj too large");
             if (fits32 && nk > 80 &&
-                launch_column<ST, CT>({uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, ext_buf,
-                                          ext_buf ? ext_bytes : row_bytes * (size_t)nj},
+                launch_column<ST, CT>({uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, ext_buf, ext_bytes,
+                                          row_bytes * (size_t)nj},
                     &rc))
                 return rc;
             void *buf = ext_buf;
             if (!ext_buf) {
-                if ((rc = scratch_for(stream, row_bytes * (size_t)nj, &buf)))
+                size_t have = 0;
+                if ((rc = scratch_for(stream, row_bytes * (size_t)nj, row_bytes * (size_t)nj, &buf, &have)))
                     return rc;
+                // (less than every row's only while the stream is captured)
+                rows = (int)std::min<size_t>((size_t)nj, have / row_bytes);
+                if (rows < 1) {
+                    set_error("gt355_vadv: a row of ni = %d, nk = %d needs %zu bytes of scratch, and the captured stream's "
+                              "buffer has %zu; run the call once outside capture first",
+                        ni, nk, row_bytes, have);
+                    return GT355_EUNSUP;
+                }
             }
             for (int j0 = 0; j0 < nj; j0 += rows) {
                 const int nr = std::min(rows, nj - j0);
