@@ -355,7 +355,9 @@ namespace gt355 {
         // the stencil phase's tables: index of the hjb settings, and the rows per wavefront each stands for
         inline int hjb_index(int hjb) { return hjb == 8 ? 0 : hjb == 32 ? 2 : 1; }
         constexpr int HJB_OF[3] = {8, 16, 32}, HROWS[3] = {1, 2, 4};
-        // FNV-1a over the batch's form, types and domain sizes: the key of its tuned configuration
+        // FNV-1a over the batch's form, types and domain sizes: the key of its tuned configuration.  The two-phase form adds
+        // a number that changes with what its settings mean, so that entries tuned on other kernels, where hjb was the
+        // rows per item (8 then, one row now), are not found.
         inline uint64_t batch_signature(int impl, int dt, int precision, const gt355_batch_domain *d, int n) {
             uint64_t h = 1469598103934665603ULL;
             auto mix = [&](int64_t v) {
@@ -364,7 +366,10 @@ namespace gt355 {
                     h *= 1099511628211ULL;
                 }
             };
+            constexpr int TWO_PHASE_KERNELS = 2;
             mix(impl), mix(dt), mix(precision), mix(n);
+            if (impl == 3)
+                mix(TWO_PHASE_KERNELS);
             for (int k = 0; k < n; ++k)
                 mix(d[k].ni), mix(d[k].nj), mix(d[k].nk), mix(d[k].phases);
             return h;
@@ -755,10 +760,11 @@ extern "C" int gt355_batch_set_config(gt355_batch *bt, const int32_t cfg[5]) {
     GT355_CHECK(bt != nullptr && cfg != nullptr, "gt355_batch_set_config: null argument");
     GT355_CHECK(cfg[0] == bt->impl, "gt355_batch_set_config: the form (%d) is fixed at create time (%d)", cfg[0],
         bt->impl);
-    GT355_CHECK(cfg[1] == 8 || cfg[1] == 16 || cfg[1] == 32, "gt355_batch_set_config: rows per item %d", cfg[1]);
-    GT355_CHECK(cfg[2] >= 1 && cfg[2] <= 8, "gt355_batch_set_config: stencil workgroups per CU %d", cfg[2]);
+    GT355_CHECK(cfg[1] == 8 || cfg[1] == 16 || cfg[1] == 32,
+        "gt355_batch_set_config: hjb %d (8, 16 or 32, once the rows per item: 1, 2 or 4 rows per wavefront)", cfg[1]);
+    GT355_CHECK(cfg[2] >= 1 && cfg[2] <= 8, "gt355_batch_set_config: hw %d (1..8; unused)", cfg[2]);
     GT355_CHECK(cfg[3] >= 1 && cfg[3] <= BWG_MAX, "gt355_batch_set_config: grid setting %d", cfg[3]);
-    GT355_CHECK(cfg[4] >= 2, "gt355_batch_set_config: deep_nk %d", cfg[4]);
+    GT355_CHECK(cfg[4] >= 2, "gt355_batch_set_config: deep_nk %d (2 or more; unused)", cfg[4]);
     bt->hjb = cfg[1];
     bt->hw = cfg[2];
     bt->w = cfg[3];

@@ -344,16 +344,16 @@ int gt355_batch_create(int precision, const gt355_batch_domain *domains, int ndo
 int gt355_batch_run(gt355_batch *batch, double dtr_stage, void *stream);
 int gt355_batch_info(const gt355_batch *batch, int *nitems, int *grid);
 /* The batch's part of the autotuner: times `reps` runs of each launch configuration (coordinate by coordinate): the
- * persistent grid setting (1..4), for FP32 storage in the two-phase form the depth from which the vertical phase
- * keeps 96 levels in registers (81, 89, 97 or never), then the stencil phase's rows per item (8, 16, 32) and
- * workgroups per CU (2, 4, 8).  It keeps the fastest for later runs of this batch, records it in the tuning table
+ * persistent grid setting (1..4), then in the two-phase form the stencil phase's rows per wavefront (1, 2 or 4, as hjb 8,
+ * 16 or 32).  It keeps the fastest for later runs of this batch, records it in the tuning table
  * under the signature of the domain list (gt355_tune_save persists it; a batch created later for the same list of
  * domain sizes, form and types starts from it), and returns the grid setting with the mean time.  The batch's
  * outputs (and utens_stage, read and rewritten by every run) are overwritten as by that many gt355_batch_run
  * calls. */
 int gt355_batch_tune(gt355_batch *batch, int reps, void *stream, int *wg_per_cu, double *best_us);
-/* The launch configuration of a batch: cfg = {form, stencil-phase rows per item, stencil-phase workgroups per CU,
- * persistent grid setting, vertical-phase 96-level depth}.  set_config applies one (the form must be the batch's). */
+/* The launch configuration of a batch: cfg = {form, hjb (8, 16 or 32: 1, 2 or 4 rows per wavefront of the stencil phase),
+ * hw (1..8), persistent grid setting, deep_nk (2 or more)}; hw and deep_nk are stored and returned, and choose nothing.
+ * set_config applies one (the form must be the batch's). */
 int gt355_batch_get_config(const gt355_batch *batch, int32_t cfg[5]);
 int gt355_batch_set_config(gt355_batch *batch, const int32_t cfg[5]);
 
