@@ -215,8 +215,10 @@ namespace gt355 {
         bool launch_column_blocks(const vadv_args<ST, CT> &a, int *rc) {
             constexpr bool F32 = sizeof(CT) == 4, S32 = sizeof(ST) == 4;
             constexpr int NB = R < 32 ? R : 32;
-            // the most wavefronts per SIMD whose registers hold the column and its rings without spills
-            constexpr int WMAX = F32 ? (R <= 32 ? 3 : 2) : R <= (S32 ? 16 : 8) ? 3 : R <= (S32 ? 40 : 32) ? 2 : 1;
+            // the most wavefronts per SIMD whose registers hold the column and its rings of 8 levels without spills (three
+            // of FP64 up to 16 levels and of the mixed form at 17 to 24 spill: 1024x1024x9 FP64 110 against 90 of two,
+            // 1024x1024x20 mixed 97 and 84)
+            constexpr int WMAX = F32 ? (R <= 32 ? 3 : 2) : R <= (S32 ? 8 : 0) ? 3 : R <= (S32 ? 40 : 32) ? 2 : 1;
             constexpr int D = !F32 && R <= 32 && R > (S32 ? 24 : 16) ? 4 : 8;
             const int64_t items = (int64_t)((a.ni + 63) / 64) * a.nj, simds = (int64_t)cu_count() * 4;
             // Wavefronts per SIMD: a round of w takes about w times a round of one, so the fewest rounds times w, as many
@@ -234,6 +236,12 @@ namespace gt355 {
             // the rounds' ends (512x512x40 FP64 77.0 and 78.8; 900x900x80 mixed 294 and 307, but 1024x1024x80 356 and 346).
             const int64_t bytes = items * 64 * a.nk * (int64_t)sizeof(ST);
             const int per_launch = w < 3 && a.nk >= 32 && bytes >= ((F32 || !S32 ? 150LL : 300LL) << 20) ? 1 : 0;
+            // there three wavefronts with 4 levels ahead, without spills, where they run all strips in one round (400x400x8
+            // FP64 10.2 against 11.6 with 8 ahead, 14.1 of two wavefronts; 360x360x12 14.3, 17.2 and 17.7; 360x360x20 mixed
+            // 13.5, 15.7 and 16.3)
+            if constexpr (!F32 && WMAX == 2 && R <= (S32 ? 16 : 8))
+                if (items > simds * 2 && items <= simds * 3)
+                    return launch_column_as<ST, CT, R, 4, 0, NB, true, false, MINK, 3>(a, 0, rc);
             if constexpr (WMAX >= 3)
                 if (w == 3)
                     return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 3>(a, per_launch, rc);
