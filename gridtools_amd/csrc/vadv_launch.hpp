@@ -236,8 +236,8 @@ namespace gt355 {
             // the rounds' ends (512x512x40 FP64 77.0 and 78.8; 900x900x80 mixed 294 and 307, but 1024x1024x80 356 and 346).
             const int64_t bytes = items * 64 * a.nk * (int64_t)sizeof(ST);
             const int per_launch = w < 3 && a.nk >= 32 && bytes >= ((F32 || !S32 ? 150LL : 300LL) << 20) ? 1 : 0;
-            // there three wavefronts with 4 levels ahead, without spills, where they run all strips in one round (400x400x8
-            // FP64 10.2 against 11.6 with 8 ahead, 14.1 of two wavefronts; 360x360x12 14.3, 17.2 and 17.7; 360x360x20 mixed
+            // Where three wavefronts spill with 8 levels ahead, three with 4, which do not, if they run all strips in one round
+            // (400x400x8 FP64 10.2 against 11.6 with 8 ahead, 14.1 of two wavefronts; 360x360x12 14.3, 17.2 and 17.7; 360x360x20 mixed
             // 13.5, 15.7 and 16.3)
             if constexpr (!F32 && WMAX == 2 && R <= (S32 ? 16 : 8))
                 if (items > simds * 2 && items <= simds * 3)
@@ -250,11 +250,12 @@ namespace gt355 {
                     return launch_column_as<ST, CT, R, (R >= 40 ? 4 : D), 0, NB, true, false, MINK, 2>(
                         a, per_launch, rc);
             // FP32 storage, one wavefront per SIMD: 4 levels ahead keep the reads in flight below what the memory takes
-            // where most SIMDs have one (256x256x80 mixed 20.4 against 22.0 with 8 ahead; 1536x1536x80 in rounds 824 against
-            // 843); 8 levels where few do (64x64x80 12.7 against 13.0) and, a little, over two to four rounds
+            // where more than three of a CU's four SIMDs have one (256x256x80 mixed 20.4 against 22.0 with 8 ahead, 832
+            // strips 18.7 and 20.1; 1536x1536x80 in rounds 824 against 843); 8 levels where fewer do (768 strips mixed 17.2
+            // against 18.3, FP32 16.7 and 17.5, 256x160x80 FP32 15.3 and 17.3) and, a little, over two to four rounds
             // (512x512x80 79.6 against 80.3, 400x400x80 54.4 against 56.0).  FP64: 8 (64x64x80 12.1 against 14.2).
             if constexpr (S32 && R >= 40)
-                if (items * 2 > simds && (items <= simds || items > simds * 4))
+                if (items * 4 > simds * 3 && (items <= simds || items > simds * 4))
                     return launch_column_as<ST, CT, R, 4, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
             // FP64, all strips at once: the neighbours' lines are shared in flight, so wcon need not stay in the caches,
             // where other stencils' fields do (hdiff and this in turn, 256x256x80: 65.7 per pair with the default policy,
