@@ -263,6 +263,11 @@ namespace gt355 {
             if constexpr (!S32 && R >= 40)
                 if (items <= simds)
                     return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 1, CPOL_NT>(a, 0, rc);
+            // (the 4 levels of load-ahead of two wavefronts per SIMD are too few where half of the SIMDs or more have no strip:
+            // 96x96x32 FP64 6.5 with 4, 6.1 with 8, over rotating fields 7.6 and 6.5; 200x200x32 12.1 and 12.2)
+            if constexpr (!S32 && R == 24)
+                if (items * 2 <= simds)
+                    return launch_column_as<ST, CT, R, 8, 0, NB, true, false, MINK, 1>(a, 0, rc);
             return launch_column_as<ST, CT, R, D, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
         }
 
