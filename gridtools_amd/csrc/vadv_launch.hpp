@@ -235,7 +235,13 @@ namespace gt355 {
             // 1536x1536x80 mixed 938 and 824, FP32 925 and 836); smaller or shallower ones lose the wavefronts' overlap at
             // the rounds' ends (512x512x40 FP64 77.0 and 78.8; 900x900x80 mixed 294 and 307, but 1024x1024x80 356 and 346).
             const int64_t bytes = items * 64 * a.nk * (int64_t)sizeof(ST);
-            const int per_launch = w < 3 && a.nk >= 32 && bytes >= ((F32 || !S32 ? 150LL : 300LL) << 20) ? 1 : 0;
+            // FP64 also where two launches have three quarters of the SIMDs or fewer each: one launch makes some wavefronts
+            // solve two strips while others solve one, and all reads compete meanwhile (one launch against two: 300x300x80 65.6
+            // and 58.7, over rotating fields 66.2 and 59.5, after hdiff 102 and 96; 256x350x56 45.8 and 40.9; 1600 strips
+            // 256x400x80 70.5 and 68.9, 256x400x44 42.3 and 42.2; 1030 strips 64x1030x80 47.1 and 51.7)
+            const bool halves = !S32 && R >= 40 && w == 1 && items * 8 >= simds * 9 && items * 2 <= simds * 3;
+            const int per_launch =
+                halves || (w < 3 && a.nk >= 32 && bytes >= ((F32 || !S32 ? 150LL : 300LL) << 20)) ? 1 : 0;
             // Where three wavefronts spill with 8 levels ahead, three with 4, which do not, if they run all strips in one round
             // (400x400x8 FP64 10.2 against 11.6 with 8 ahead, 14.1 of two wavefronts; 360x360x12 14.3, 17.2 and 17.7; 360x360x20 mixed
             // 13.5, 15.7 and 16.3)
