@@ -111,9 +111,12 @@ namespace gt355 {
         if (mib < 36)
             return st_size == 4 ? hdiff_cfg{2, 4, 8, 1} : hdiff_cfg{2, 2, 6, 1};
         // FP64 past the caches: pairs, 4 rows (512x512x80 82.2 against 87.2 of 8 rows, 300x700x90 76.7 against 79.8 of the
-        // one-column sweep, 1000x1000x80 307 and 315; 384x384x80, 270 MiB, 47.5 and 46.9)
+        // one-column sweep, 1000x1000x80 307 and 315; 384x384x80, 270 MiB, 47.5 and 46.9), but the flat pair sweep where the
+        // strips fill less than 60% of their lanes (pairs / flat / one column per lane: 130x1890x80 89 / 75 / 85 on one set
+        // of fields, 96 / 87 / 93 over rotating ones, 140x2730x80 132 / 113 / 126, 143 / 133 / 138; pairs / flat at 31%
+        // 40x5734x80 120 / 75, 125 / 88, at 63% 80x4096x80 101 / 98, 113 / 115, at 68% 260x1260x80 96 / 94, 109 / 110)
         if (st_size == 8 && mib >= 400)
-            return hdiff_cfg{2, 4, 4, 0};
+            return 10 * (int64_t)ni < 6 * (((int64_t)ni + 127) / 128 * 128) ? hdiff_cfg{2, 4, 8, 1} : hdiff_cfg{2, 4, 4, 0};
         // Where many lanes of the strips would idle, the flat pair sweep: below 95% filled for FP32 storage (300x300x80
         // mixed 18.0 against 19.9, 130x400x137 19.7 against 26.2; at 98%, 1000x1000x80 FP32, 184-187 against 177), below
         // 80% for FP64 (130x400x137 30.8 against 33.1; at 86%, 387x251x61, 26.0 against 25.2)
