@@ -302,9 +302,21 @@ namespace gt355 {
                         // the other dimension: lines of 128 bytes, as many as make a tile of about 1024 elements (a
                         // shorter tile leaves a workgroup of 256 idle: 500x500x20 FP64 80 us with one line, 35 with
                         // four; longer ones take more LDS: 197x261x73 28.4, 29.9, 35.0 us with 16, 32, 64 elements)
-                        constexpr int A = 128 / (int)sizeof(W), V = sizeof(W) >= 4 ? 16 / (int)sizeof(W) : 1;
-                        const int cut = (int)std::min<int64_t>(
-                            std::max(na, nb), A * ((1024 + A * run - 1) / (A * run)));
+                        constexpr int V = sizeof(W) >= 4 ? 16 / (int)sizeof(W) : 1;
+                        const int64_t other = std::max(na, nb);
+                        auto cut_of = [&](int a) { return (int)std::min<int64_t>(other, a * ((1024 + a * run - 1) / (a * run))); };
+                        int cut = cut_of(128 / (int)sizeof(W));
+                        // elements of 1 and 2 bytes move one per access, so a tile of whole lines is up to eight times the
+                        // work: half lines of 1 byte for longer runs (500x500x65 49.8 -> 44.4 us over rotating buffers, x16
+                        // 13.4 and 15.7), and shorter pieces yet while there are fewer than four tiles per CU (1 byte
+                        // 97x131x73 12.3 -> 6, 128x128x137 23 / 14 / 9.6 / 8.2 in pieces of 128 / 64 / 32 / 16; 2 bytes
+                        // 128x128x80 9.7 / 7.6 / 6.7 in 64 / 32 / 16; 256x256x65, 1024 tiles, 12.4 / 13.0 / 15.3)
+                        if constexpr (sizeof(W) < 4)
+                            for (int a = sizeof(W) == 1 && run <= 32 ? 128 : 64; a >= 16; a /= 2) {
+                                cut = cut_of(a);
+                                if ((other + cut - 1) / cut * outer >= 1024)
+                                    break;
+                            }
                         const int ta = na <= nb ? (int)run : cut, tb = na <= nb ? cut : (int)run;
                         const int64_t tiles_a = (na + ta - 1) / ta, tiles_b = (nb + tb - 1) / tb,
                                       ntiles = tiles_a * tiles_b * outer;
