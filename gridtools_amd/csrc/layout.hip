@@ -321,19 +321,27 @@ namespace gt355 {
                         const int64_t tiles_a = (na + ta - 1) / ta, tiles_b = (nb + tb - 1) / tb,
                                       ntiles = tiles_a * tiles_b * outer;
                         // 16-byte accesses on a side whose tile rows all start 16-byte aligned
-                        auto side = [&](const void *p, const int64_t *st, int unit, int ext, int64_t full) {
-                            if (V == 1 || !vec_on || st[unit] != 1 || (uintptr_t)p % 16 || (ext < full && ext % V))
+                        auto rows_on = [&](int bytes, const void *p, const int64_t *st, int unit) {
+                            if ((uintptr_t)p % bytes)
                                 return false;
                             for (int q = 0; q < d.nd; ++q)
-                                if (q != unit && d.dims[q] > 1 && (st[q] * (int64_t)sizeof(W)) % 16)
+                                if (q != unit && d.dims[q] > 1 && (st[q] * (int64_t)sizeof(W)) % bytes)
                                     return false;
                             return true;
+                        };
+                        auto side = [&](const void *p, const int64_t *st, int unit, int ext, int64_t full) {
+                            return V > 1 && vec_on && st[unit] == 1 && (ext == full || ext % V == 0) &&
+                                   rows_on(16, p, st, unit);
                         };
                         const bool va = side(src, d.ss, d.a, ta, na), vb = side(dst, d.ds, d.b, tb, nb);
                         // whole lines of arrays past what the Infinity Cache would keep for the next call are streams
                         // (301x303x137 FP64 86 -> 73 us non-temporal, 256x256x80 35.9 -> 37.5), and their tiles go to the XCDs in
-                        // groups (512x512x80 FP64 135 -> 128 us, FP32 75 -> 73; 197x261x73 FP64, not one, 28.5 -> 30.0)
-                        const bool nt = (int64_t)sizeof(W) * na * nb * outer >= (int64_t(64) << 20);
+                        // groups (512x512x80 FP64 135 -> 128 us, FP32 75 -> 73; 197x261x73 FP64, not one, 28.5 -> 30.0).
+                        // Not where rows are written 16 bytes at a time that do not start on lines: a non-temporal store
+                        // of part of a line does not wait for the rest of it (FP64 from k-fastest into rows of 506 elements,
+                        // 500x500x160 268 us non-temporal, 185 else; 300x300x100 59 and 21, over rotating buffers 62 and 38)
+                        const bool nt = (int64_t)sizeof(W) * na * nb * outer >= (int64_t(64) << 20) &&
+                                        (!vb || rows_on(128, dst, d.ds, d.b));
                         auto magic = [](int n) { return n == 1 ? 0u : (uint32_t)(((uint64_t(1) << 32) + n - 1) / n); };
                         if (ntiles <= (int64_t(1) << 23)) { // one workgroup per tile
                             const uint32_t ma = magic(va ? (ta + V - 1) / V : ta), mb = magic(vb ? (tb + V - 1) / V : tb);
