@@ -32,7 +32,7 @@
 
 namespace gt355 {
     namespace {
-        constexpr int BTI = 64, BTJ = 4, BMAXK = 144;
+        constexpr int BTI = 64, BTJ = 4, BMAXK = VMAXK;
         // forward steps run up to D-1 levels past a column's top; scratch rows = deepest nk + BPAST
         constexpr int BPAST = 8;
 
@@ -331,7 +331,7 @@ struct gt355_batch {
     void *hitems[3];  // and, with each, the hitems of the domains that its flat sweep does not take
     void *scratch; // ccol/dcol of every workgroup the grid may have, in the compute type
     int impl;      // 1: 64x4 tiles, ccol/dcol in scratch; 2: 64-column strips, ccol/dcol in registers;
-                   // 3: two phases (stencil sweep, then the vertical advection over column-list items)
+                   // 3: two phases (stencil sweep, then the vertical advection over 64-column strips)
     int nk_reg;    // strip form: levels of ccol/dcol held in registers (80: one wavefront per SIMD; 32: two)
     vertical_plan plan; // two-phase form: the vertical items' depth classes
     int deep_nk;   // a value of the stored configurations that no kernel reads any more
@@ -528,9 +528,9 @@ int gt355::batch_create_form(int precision, const gt355_batch_domain *domains, i
     batch_cfg cfg{16, 8, wg_per_cu, 89};
     (void)find_batch_cfg(bt->sig, dt == GT355_F64 ? 8 : 4, batch_ct(bt), impl, &cfg);
     bt->hjb = HJB_OF[hjb_index(tune_param("batch_hjb", cfg.hjb))];
-    bt->hw = std::min(8, std::max(1, tune_param("batch_hw", cfg.hw)));
+    bt->hw = std::min(8, std::max(1, cfg.hw));
     bt->w = std::min(BWG_MAX, std::max(1, cfg.w));
-    bt->deep_nk = tune_param("batch_deep_nk", cfg.deep_nk);
+    bt->deep_nk = cfg.deep_nk;
     bt->grid = batch_grid(bt, bt->w);
     bt->gridmax = batch_grid(bt, BWG_MAX); // scratch for any grid the tuner may pick
     const size_t item_bytes = impl >= 2 ? sizeof(sitem) * sitems.size() : sizeof(bitem) * items.size();

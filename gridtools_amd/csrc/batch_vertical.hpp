@@ -25,9 +25,9 @@ namespace gt355 {
 
     // The items' depth classes, deepest first: class n takes depths above vertical_above(n) up to the class before it.
     constexpr int VCLASSES = 8;
-    // levels past the deepest split's registers and LDS (128, or 104 where no column is deeper than 112) that a wavefront
-    // of the vertical phase may keep in its scratch, up to 144 levels
-    constexpr int VTAIL_ROWS = 16;
+    // Depths of at most VMAXK; the levels below the top block of 8 that a wavefront of the vertical phase keeps in its
+    // scratch, past the 128 that the deepest split (FP64 arithmetic, from 81 or 113 levels) has in registers and LDS.
+    constexpr int VMAXK = 144, VTAIL_ROWS = (VMAXK - 128 - 1) / 8 * 8;
     struct vertical_plan {
         int end[VCLASSES]; // items are sorted by class: those of class n end here
     };

@@ -178,17 +178,6 @@ namespace gt355 {
                 __builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b128(r, 0, 0, 0)), v), r, voff, soff,
                 CPOL);
     }
-    // 16 bytes per lane (four FP32 elements, i to i+3) in one request
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    template <int CPOL = 0>
-    __device__ __forceinline__ f32x4 bload4(rsrc_t r, uint32_t voff, uint32_t soff) {
-        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, CPOL));
-    }
-    template <int CPOL = 0>
-    __device__ __forceinline__ void bstore4(rsrc_t r, f32x4 v, uint32_t voff, uint32_t soff) {
-        __builtin_amdgcn_raw_buffer_store_b128(
-            __builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b128(r, 0, 0, 0)), v), r, voff, soff, CPOL);
-    }
     template <class T, int CPOL = 0>
     __device__ __forceinline__ void bstore(rsrc_t r, T v, uint32_t voff, uint32_t soff) {
         if constexpr (sizeof(T) == 4)
