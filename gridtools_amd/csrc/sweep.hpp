@@ -133,8 +133,8 @@ namespace gt355 {
     // scalar loads.  flx at b-1 is flx at a, so each lane evaluates three x-fluxes, not four.  Lanes past the
     // domain load the last pair (clamped) and store nothing; since ni is even, the lane after the last valid
     // one loads exactly columns ni and ni+1, the right neighbours the last valid lane needs.  The launcher uses
-    // it for even ni with 2-element-aligned rows (origin and j/k strides); other shapes take the one-column
-    // sweep.
+    // it for even ni with 2-element-aligned rows (origin and j/k strides); other shapes take the flat sweep below (FP32
+    // storage) or the one-column sweep (FP64).
     // The wavefront's strip is columns [i0, i0+128) x rows [j0, j0+JB) of level k (wave-uniform); LAP also stores the
     // laplacian of every output point into `lap`, laid out like `out`.  PO / PI as for hdiff_sweep_wave.
     template <class ST, class CT, int JB, int P, bool LAP, class PO = ST *, class PI = const ST *>
@@ -253,11 +253,13 @@ namespace gt355 {
     // sides, and a lane's flx at its left edge is the left lane's flx (a shift instead of a fourth flux).  Rows of any
     // width fill their lanes, and an odd ni or unaligned rows need no more than the last pair's handling below (a
     // request only needs element alignment).
-    // What bounds it: ~28 vector instructions per point against ~78 of the one-column sweep (mixed form), so requests:
-    // a wavefront's rows start anywhere, five lines where an aligned 128-column strip has four.  Full strips therefore
-    // stay with hdiff_pair_wave (512x512x80 FP64 82 us against 85 here, 1536x1536x80 mixed 382 against 394)
-    // and ragged widths come here (mixed, us, strips / flat: 387x251x61 19.6 / 16.2, 130x400x137 26.2 / 19.7,
-    // 101x203x60 8.3 / 5.9).  All JB + 4 = 8 rows are loaded ahead: one memory latency per wavefront.
+    // What bounds it: ~28 vector instructions per point against ~78 of the one-column sweep (mixed form), so not those but
+    // what is in flight: all JB + 4 rows (JB 4, 2 or 1) are loaded ahead, so a wavefront waits for memory once, and has
+    // nothing in flight while it computes and stores; 7 wavefronts per SIMD cover for that in part (387x251x61 mixed 4.4
+    // TB/s, like the aligned 256x256x80 on strips; about 5 us of it a launch's ramp and drain).  A wavefront's rows start
+    // anywhere, five lines where an aligned 128-column strip has four: full strips stay with hdiff_pair_wave
+    // (512x512x80 FP64 82 us against 85 here, 1536x1536x80 mixed 382 against 394) and ragged widths come here (mixed, us,
+    // strips / flat: 387x251x61 19.6 / 16.2, 130x400x137 26.2 / 19.7, 101x203x60 8.3 / 5.9).
     // Rows: block b covers output rows b*JB.., moved up to end at nj (j0 = min(b*JB, nj - JB), nj >= JB); rows that the
     // block before owns are computed but not stored, so every row has one writer.  Addresses are buffer descriptors
     // plus a lane offset and one scalar offset per row (the launcher checks that every field spans less than 4 GiB).

@@ -99,8 +99,8 @@ namespace gt355 {
         // consecutive) with a static stride, so that the wavefronts in flight stay on neighbouring strips.  Each starts
         // the next strip's first D levels of loads NB levels before the end of a strip's backward sweep, so the next
         // forward sweep needs no pipeline fill.  Measured against the former kernels (one level bucket per 16 levels,
-        // selects at every level), us: 256x256x80 FP64 37.7 (39.7), mixed 20.4 (21.7); 64x64x80 FP64 12.1 (15.5), mixed
-        // 12.7 (16.3), FP32 10.4 (13.3); 512x512x40 mixed 40.6 (54.2); 192x160x137 FP64 35.1 (124 through memory).
+        // selects at every level), us: 256x256x80 FP64 37.7 (39.7), mixed 20.4 (21.7); 300x300x40 FP64 28
+        // (38), FP32 17 (22); 512x512x40 mixed 40.6 (54.2); 300x300x137 FP64 128 (209 through memory).
         template <class ST, class CT, int R, int D, int TL, int NB, bool PARK, bool DEEP, int MINK, int WPE, int CPOL_W>
         __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
         vadv_column_kernel(ST *__restrict__ uts_f, const ST *__restrict__ us_f, const ST *__restrict__ wc_f,
@@ -259,7 +259,8 @@ namespace gt355 {
             // where more than three of a CU's four SIMDs have one (256x256x80 mixed 20.4 against 22.0 with 8 ahead, 832
             // strips 18.7 and 20.1; 1536x1536x80 in rounds 824 against 843); 8 levels where fewer do (768 strips mixed 17.2
             // against 18.3, FP32 16.7 and 17.5, 256x160x80 FP32 15.3 and 17.3) and, a little, over two to four rounds
-            // (512x512x80 79.6 against 80.3, 400x400x80 54.4 against 56.0).  FP64: 8 (64x64x80 12.1 against 14.2).
+            // (512x512x80 79.6 against 80.3, 400x400x80 54.4 against 56.0).  FP64: 8 (64x64x80 on
+            // one wavefront per strip 12.1 against 14.2).
             if constexpr (S32 && R >= 40)
                 if (items * 4 > simds * 3 && (items <= simds || items > simds * 4))
                     return launch_column_as<ST, CT, R, 4, 0, NB, true, false, MINK, 1>(a, per_launch, rc);
@@ -349,6 +350,7 @@ namespace gt355 {
             const bool fits32 = span < (int64_t(1) << 32);
             int rc = GT355_OK;
             if (fits32 && nk <= 80) {
+                // (a limit of the calls, not of this kernel, whose grid is one-dimensional: what it refuses stays refused)
                 GT355_CHECK(nj <= 65535, "gt355_vadv: nj too large");
                 if (launch_column<ST, CT>({uts, us, wc, up, ut, dtr_c, ni, nj, nk, stream, nullptr, 0, 0}, &rc))
                     return rc;
