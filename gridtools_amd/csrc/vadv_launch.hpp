@@ -230,6 +230,10 @@ namespace gt355 {
             for (int v = WMAX - 1; v >= 1; --v)
                 if (rounds(v) * v * 8 < rounds(w) * w * 7)
                     w = v;
+            // (FP64 of 9 to 16 levels over many rounds: one, which starts its next strip's loads sooner; 1400x1400x12 189
+            // against 197 of two, over rotating fields 213 and 223, 1024x1024x9 87 and 90; 700x700x9, 7.5 strips per SIMD, 45 and 45)
+            if (!S32 && R == 8 && MINK > 8 && items > simds * 12)
+                w = 1;
             // A launch per round for large fields: over many rounds in one launch the wavefronts drift apart, and the
             // memory with them (one launch against one per round: 512x512x80 FP64 161 and 152, 1024x1024x80 744 and 686,
             // 1536x1536x80 mixed 938 and 824, FP32 925 and 836); smaller or shallower ones lose the wavefronts' overlap at

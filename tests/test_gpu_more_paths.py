@@ -17,6 +17,13 @@ def test_column_sweep_block_edges(gpu, oracle, nk, dtype, precision, mode):
     _check(gpu, oracle, 65, 300, nk, dtype, precision, mode)
 
 
+@pytest.mark.parametrize("nj", [6144, 6145])  # two strips per row: 12 strips per SIMD on 256 CUs, and more
+@pytest.mark.parametrize("nk", [8, 9, 16])
+def test_many_strips(gpu, oracle, nk, nj):
+    """One wavefront per SIMD for FP64 of 9 to 16 levels past 12 strips per SIMD."""
+    _check(gpu, oracle, 65, nj, nk, np.float64, 0, "native")
+
+
 def _inf_fields(ni, nj, nk, dtype):
     rng = np.random.default_rng(ni * 7 + nk)
     shp = (nk, nj + 2 * H, ni + 2 * H)
