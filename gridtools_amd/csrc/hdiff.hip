@@ -215,7 +215,9 @@ namespace gt355 {
         // The sweeps' XCD mapping: groups where the three fields take at least `mib` MiB.  The strips from 256 MiB, past
         // the Infinity Cache (1536x1536x80 mixed 402 us in eighths, 389 in groups; 1000x1000x60 136 and 132); the flat
         // pair sweep from 32 MiB (387x251x61 mixed 16.5 and 16.2, 300x300x80 18.9 and 18.0; 101x203x60, 15 MiB, 5.9
-        // and 6.0).
+        // and 6.0).  These are fields that other calls' fields have displaced from the caches, as in a timestep; the same
+        // fields again and again lose up to 1 GiB, since eighths keep more of them in the Infinity Cache (FP32 520x945x80,
+        // 450 MiB, 70.4 and 73.1, over rotating fields 88.2 and 83.3; FP64 520x472x80 69.5 and 71.8, 83.3 and 78.2).
         int hdiff_group(int ni, int nj, int nk, size_t es, int64_t mib) {
             return 3 * (int64_t)ni * nj * nk * (int64_t)es >= mib << 20 ? XCD_GROUP : 0;
         }
